@@ -608,27 +608,28 @@ int tension_decode_step(const tension_buf* q, const tension_buf* k_new, const te
   };
   auto all16 = [&](int32_t dt) {
     return a16(q, false, dt) && a16(k_new, false, dt) && a16(v_new, false, dt) && a16(out, false, dt) &&
-           a16(k_cache, true, dt) && a16(v_cache, true, dt) && slab_fits(k_cache, 2) && slab_fits(v_cache, 2);
+           a16(k_cache, true, dt) && a16(v_cache, true, dt);
   };
-  const bool f32qk = a32(q, false) && a32(k_new, false) && a32(out, false) && a32(k_cache, true) &&
-                     slab_fits(k_cache, 4);
-  int flow = DECODE_EXACT;
-  if (!(flags & TENSION_FORCE_EXACT) && D == 64 && W <= 1024) {
-    if (all16(TENSION_BF16)) {
-      flow = DECODE_BF16;
-    } else if (all16(TENSION_F16)) {
-      flow = DECODE_F16;
-    } else if (f32qk && !(flags & TENSION_DECODE_SELF)) {
-      // the reference's autocast flow: float32 q / K (promoted by RoPE), bf16
-      // V; or float32 throughout (no autocast)
-      if (a16(v_new, false, TENSION_BF16) && a16(v_cache, true, TENSION_BF16) && slab_fits(v_cache, 2))
-        flow = DECODE_KF32;
-      else if (W <= 512 && a32(v_new, false) && a32(v_cache, true) && slab_fits(v_cache, 4))
-        flow = DECODE_F32;
-    }
+  // the element types, when every row is 16-byte aligned
+  int rows = DECODE_EXACT;
+  if (all16(TENSION_BF16)) {
+    rows = DECODE_BF16;
+  } else if (all16(TENSION_F16)) {
+    rows = DECODE_F16;
+  } else if (a32(q, false) && a32(k_new, false) && a32(out, false) && a32(k_cache, true)) {
+    // the reference's autocast flow: float32 q / K (promoted by RoPE), bf16
+    // V; or float32 throughout (no autocast)
+    if (a16(v_new, false, TENSION_BF16) && a16(v_cache, true, TENSION_BF16)) rows = DECODE_KF32;
+    else if (a32(v_new, false) && a32(v_cache, true)) rows = DECODE_F32;
   }
+  if ((flags & TENSION_FORCE_EXACT) || (D != 32 && D != 64 && D != 128)) rows = DECODE_EXACT;
+  // the fast kernel: head dim 64, W <= 1024 (float32 throughout: 512), 16-bit
+  // rows for the self-key step, slabs that fit its descriptors
+  const int ek = k_cache->dtype == TENSION_F32 ? 4 : 2, ev = v_cache->dtype == TENSION_F32 ? 4 : 2;
+  const bool fast = rows != DECODE_EXACT && D == 64 && W <= (rows == DECODE_F32 ? 512 : 1024) &&
+                    !((flags & TENSION_DECODE_SELF) && ek == 4) && slab_fits(k_cache, ek) && slab_fits(v_cache, ev);
   hipError_t e = hipSuccess;
-  launch_decode(flow, is_f64(q) || is_f64(k_cache) || is_f64(v_cache), p, hs(stream), &e);
+  launch_decode(fast ? rows : DECODE_EXACT, rows, is_f64(q) || is_f64(k_cache) || is_f64(v_cache), p, hs(stream), &e);
   return launched(e, "tension_decode_step");
 }
 

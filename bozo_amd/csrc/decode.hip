@@ -6,6 +6,8 @@
 // loads before any arithmetic, eight lanes cover one 128-byte cache row (1 KB
 // of contiguous cache per wave load instruction), and the sums are folded with
 // DPP lane moves and one LDS pass.
+#include <type_traits>
+
 #include "kernels.h"
 
 namespace tension {
@@ -330,62 +332,224 @@ __global__ __launch_bounds__(64 * NW) void decode_d64(DecodeFastArgs p) {
   decode_d64_body<NW, NP, FLOW, SELF>(p);
 }
 
-// Exact path: any dtype, any D <= 256, any W; one thread per (n, h).  The
-// thread reads every slot before it overwrites slot pos % W, so the
-// read-before-write order holds within the thread.
-template <typename A>
-__global__ __launch_bounds__(64) void decode_exact(DecodeParams p) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= p.N * p.H) return;
-  const int n = idx / p.H, h = idx % p.H;
-  const int pos = p.pos_in[n] > 0 ? p.pos_in[n] : 0;
-  const int W = p.W, D = p.D;
-  const A scale = (A)p.scale;
-  A acc[256];
-  for (int d = 0; d < D; ++d) acc[d] = A(0);
-  A msum = A(0);
-  const int64_t qo = n * p.q.s0 + h * p.q.s1;
-  for (int slot = 0; slot < W; ++slot) {
-    const bool ok = pos >= W || slot < pos;
-    A tau = A(0);
-    if (ok) {
-      const int64_t ko = n * p.kc.s0 + h * p.kc.s1 + (int64_t)slot * p.kc.s2;
-      const int64_t vo = n * p.vc.s0 + h * p.vc.s1 + (int64_t)slot * p.vc.s2;
-      A dot = A(0);
-      for (int d = 0; d < D; ++d) dot += ld<A>(p.q, qo + d) * ld<A>(p.kc, ko + d);
-      tau = sigmoid_exact(dot / scale);
-      for (int d = 0; d < D; ++d) acc[d] += tau * ld<A>(p.vc, vo + d);
-    }
-    msum += tau;
-    if (p.tau.p) st<A>(p.tau, n * p.tau.s0 + h * p.tau.s1 + ring_w(slot, pos, W), tau);
+// Every other decode step (head dims other than 64, the float32 self-key step
+// of a global layer's cache, caches past the fast path's length, mixed or
+// unaligned rows).  One workgroup owns one (n, h): LPR lanes cover a cache row
+// and 64 / LPR rows go through a wave at a time, so the step is as parallel
+// over its keys as over its sequences; only live rows are read (all W slots
+// when tau is written, whose empty slots are zeros).  Bound by HBM like the
+// fast path.  libm exp and IEEE division, sums in A.  N16 H12 D64, 700 of
+// 1024 slots live, float32 self-key: 17.4 ms with one thread per (n, h).
+
+// One wave's row dot product over LPR lanes (a power of two, at most 64).
+template <int LPR, typename A>
+__device__ __forceinline__ A lanes_sum(A x) {
+#pragma unroll
+  for (int m = 1; m < LPR; m <<= 1) x += __shfl_xor(x, m);
+  return x;
+}
+
+// The step's end, shared by the kernels below: lane row groups and waves meet
+// in LDS, the output row goes out normalised and the new token's rows enter
+// the ring.  acc[e] is feature feat(e) of the lane's partial sums (the same
+// features on every lane with the same lane % LPR).
+template <int LPR, int NW, int NE, typename A, typename Feat>
+__device__ __forceinline__ void decode_finish(const DecodeParams& p, int n, int h, int pos, int live, bool self_key,
+                                              A* acc, A msum, A* red, A* mred, Feat feat) {
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int D = p.D;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+#pragma unroll
+    for (int m = LPR; m < 64; m <<= 1) acc[e] += __shfl_xor(acc[e], m);
   }
-  const int64_t no = n * p.kn.s0 + h * p.kn.s1;
-  const int64_t nvo = n * p.vn.s0 + h * p.vn.s1;
-  const bool self_key = (p.flags & TENSION_DECODE_SELF) != 0;
-  if (self_key) {  // the new token as a key (s <= t)
-    A dot = A(0);
-    for (int d = 0; d < D; ++d) dot += ld<A>(p.q, qo + d) * ld<A>(p.kn, no + d);
-    const A tau = sigmoid_exact(dot / scale);
-    for (int d = 0; d < D; ++d) acc[d] += tau * ld<A>(p.vn, nvo + d);
-    msum += tau;
+#pragma unroll
+  for (int m = LPR; m < 64; m <<= 1) msum += __shfl_xor(msum, m);
+  if (lane < LPR) {
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+      if (feat(e) < D) red[wave * D + feat(e)] = acc[e];
+    if (lane == 0) mred[wave] = msum;
   }
+  __syncthreads();  // every cache read of this (n, h) is complete past here
+  A m = A(0);
+#pragma unroll
+  for (int w = 0; w < NW; ++w) m += mred[w];
   A inv = A(1);
   if (p.flags & TENSION_NORM_MASS) {
-    inv = A(1) / (msum > A(kMassEps) ? msum : A(kMassEps));
+    inv = A(1) / (m > A(kMassEps) ? m : A(kMassEps));
   } else if (p.flags & TENSION_NORM_COUNT) {
-    const int keys = (pos < W ? pos : W) + (self_key ? 1 : 0);
+    const int keys = live + (self_key ? 1 : 0);
     inv = A(1) / A(keys > 1 ? keys : 1);
   }
-  const int64_t oo = n * p.out.s0 + h * p.out.s1;
-  for (int d = 0; d < D; ++d) st<A>(p.out, oo + d, acc[d] * inv);
-  const int slot = pos % W;
-  const int64_t ko = n * p.kc.s0 + h * p.kc.s1 + (int64_t)slot * p.kc.s2;
-  const int64_t vo = n * p.vc.s0 + h * p.vc.s1 + (int64_t)slot * p.vc.s2;
-  for (int d = 0; d < D; ++d) {
-    st<A>(p.kc, ko + d, ld<A>(p.kn, no + d));
-    st<A>(p.vc, vo + d, ld<A>(p.vn, nvo + d));
+  const int slot = pos % p.W;
+  for (int d = tid; d < D; d += 64 * NW) {
+    A o = A(0);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) o += red[w * D + d];
+    st<A>(p.out, n * p.out.s0 + h * p.out.s1 + d, o * inv);
+    st<A>(p.kc, n * p.kc.s0 + h * p.kc.s1 + (int64_t)slot * p.kc.s2 + d, ld<A>(p.kn, n * p.kn.s0 + h * p.kn.s1 + d));
+    st<A>(p.vc, n * p.vc.s0 + h * p.vc.s1 + (int64_t)slot * p.vc.s2 + d, ld<A>(p.vn, n * p.vn.s0 + h * p.vn.s1 + d));
   }
-  if (h == 0 && p.pos_out) p.pos_out[n] = pos + 1;
+  if (tid == 0 && h == 0 && p.pos_out) p.pos_out[n] = pos + 1;
+}
+
+// 16-byte aligned rows of 8 LPR elements: a lane holds 8 consecutive features
+// and keeps U rows of K and V in flight ahead of the U it works on.  QT: q,
+// k_new, the K cache and out; VT: v_new and the V cache.
+template <typename T>
+struct Row8 {
+  u16x8 a, b;  // b: the second half of a float32 row piece
+};
+
+template <typename T>
+__device__ __forceinline__ Row8<T> row8_load(const T* p) {
+  Row8<T> r;
+  r.a = __builtin_nontemporal_load((const u16x8*)p);
+  if constexpr (sizeof(T) == 4) r.b = __builtin_nontemporal_load((const u16x8*)(p + 4));
+  return r;
+}
+
+template <typename T>
+__device__ __forceinline__ void row8_f32(const Row8<T>& r, float* x) {
+  if constexpr (sizeof(T) == 4) {
+    const f32x4 a = __builtin_bit_cast(f32x4, r.a), b = __builtin_bit_cast(f32x4, r.b);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x[e] = a[e];
+      x[4 + e] = b[e];
+    }
+  } else if constexpr (std::is_same<T, f16>::value) {
+    const f16x8 a = __builtin_bit_cast(f16x8, r.a);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = (float)a[e];
+  } else {
+    const bf16x8 a = __builtin_bit_cast(bf16x8, r.a);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = (float)a[e];
+  }
+}
+
+constexpr int kRowsNW = 8;  // waves per workgroup of decode_rows
+
+template <typename QT, typename VT, int LPR>
+__global__ __launch_bounds__(64 * kRowsNW) void decode_rows(DecodeParams p) {
+  constexpr int NW = kRowsNW, U = 4, RPW = 64 / LPR;
+  __shared__ float red[NW * 8 * LPR], mred[NW];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int ch = lane % LPR;
+  const int n = blockIdx.x / p.H, h = blockIdx.x % p.H, W = p.W;
+  const int pos = p.pos_in[n] > 0 ? p.pos_in[n] : 0;
+  const int live = pos < W ? pos : W;
+  const int rows = p.tau.p ? W : live;
+  const bool self_key = (p.flags & TENSION_DECODE_SELF) != 0;
+  const float scale = (float)p.scale;
+  float q[8];
+  row8_f32(row8_load((const QT*)p.q.p + n * p.q.s0 + h * p.q.s1 + 8 * ch), q);
+  const QT* kb = (const QT*)p.kc.p + n * p.kc.s0 + h * p.kc.s1 + 8 * ch;
+  const VT* vb = (const VT*)p.vc.p + n * p.vc.s0 + h * p.vc.s1 + 8 * ch;
+  // rows s0 + u RPW NW of one trip (past the cache: its last row, unused)
+  auto load = [&](int s0, Row8<QT>* k, Row8<VT>* v) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = s0 + u * RPW * NW;
+      const int64_t r = s < W ? s : W - 1;
+      k[u] = row8_load(kb + r * p.kc.s2);
+      v[u] = row8_load(vb + r * p.vc.s2);
+    }
+  };
+  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0}, msum = 0.f;
+  auto tau_of = [&](const Row8<QT>& k) __attribute__((always_inline)) {
+    float x[8], dot = 0.f;
+    row8_f32(k, x);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dot += q[e] * x[e];
+    return sigmoid_exact(lanes_sum<LPR>(dot) / scale);
+  };
+  auto add = [&](float tau, const Row8<VT>& v) __attribute__((always_inline)) {
+    float x[8];
+    row8_f32(v, x);
+    msum += tau;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] += tau * x[e];
+  };
+  const int first = wave * RPW + lane / LPR, trip = RPW * NW * U;
+  Row8<QT> k[U], kn[U];
+  Row8<VT> v[U], vn[U];
+  if (rows > 0) load(first, k, v);
+  for (int base = 0; base < rows; base += trip) {
+    const bool more = base + trip < rows;
+    if (more) load(base + trip + first, kn, vn);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = base + first + u * RPW * NW;
+      const float t = tau_of(k[u]);
+      // a dead slot's row (never a token's) is left out, not multiplied by 0
+      if (s < live) add(t, v[u]);
+      if (p.tau.p && ch == 0 && s < W)
+        st<float>(p.tau, n * p.tau.s0 + h * p.tau.s1 + ring_w(s, pos, W), s < live ? t : 0.f);
+    }
+    if (more) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        k[u] = kn[u];
+        v[u] = vn[u];
+      }
+    }
+  }
+  if (self_key && wave == 0) {  // the new token as a key: row group 0 of wave 0
+    const float t = tau_of(row8_load((const QT*)p.kn.p + n * p.kn.s0 + h * p.kn.s1 + 8 * ch));
+    const Row8<VT> sv = row8_load((const VT*)p.vn.p + n * p.vn.s0 + h * p.vn.s1 + 8 * ch);
+    if (lane < LPR) add(t, sv);
+  }
+  decode_finish<LPR, NW, 8>(p, n, h, pos, live, self_key, acc, msum, red, mred, [&](int e) { return 8 * ch + e; });
+}
+
+// Any dtypes, alignment and D <= 256: 16 lanes per row, lane l holds features
+// l, l + 16, ...
+template <typename A>
+__global__ __launch_bounds__(256) void decode_any(DecodeParams p) {
+  constexpr int LPR = 16, NW = 4, NE = 16, RPW = 64 / LPR;
+  __shared__ A red[NW * 256], mred[NW];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int ch = lane % LPR, D = p.D;
+  const int n = blockIdx.x / p.H, h = blockIdx.x % p.H, W = p.W;
+  const int pos = p.pos_in[n] > 0 ? p.pos_in[n] : 0;
+  const int live = pos < W ? pos : W;
+  const int rows = p.tau.p ? W : live;
+  const bool self_key = (p.flags & TENSION_DECODE_SELF) != 0;
+  const A scale = (A)p.scale;
+  A q[NE], acc[NE], msum = A(0);
+  const int64_t qo = n * p.q.s0 + h * p.q.s1;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int d = ch + LPR * e;
+    q[e] = d < D ? ld<A>(p.q, qo + d) : A(0);
+    acc[e] = A(0);
+  }
+  auto visit = [&](const Buf& kb, int64_t ko, const Buf& vb, int64_t vo, bool on) -> A {
+    A dot = A(0);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      const int d = ch + LPR * e;
+      if (on && d < D) dot += q[e] * ld<A>(kb, ko + d);
+    }
+    const A tau = on ? sigmoid_exact(lanes_sum<LPR>(dot) / scale) : A(0);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      const int d = ch + LPR * e;
+      if (on && d < D) acc[e] += tau * ld<A>(vb, vo + d);
+    }
+    msum += tau;
+    return tau;
+  };
+  const int64_t ko = n * p.kc.s0 + h * p.kc.s1, vo = n * p.vc.s0 + h * p.vc.s1;
+  for (int s = wave * RPW + lane / LPR; s < rows; s += RPW * NW) {
+    const A tau = visit(p.kc, ko + (int64_t)s * p.kc.s2, p.vc, vo + (int64_t)s * p.vc.s2, s < live);
+    if (p.tau.p && ch == 0) st<A>(p.tau, n * p.tau.s0 + h * p.tau.s1 + ring_w(s, pos, W), tau);
+  }
+  if (self_key && tid < LPR) visit(p.kn, n * p.kn.s0 + h * p.kn.s1, p.vn, n * p.vn.s0 + h * p.vn.s1, true);
+  decode_finish<LPR, NW, NE>(p, n, h, pos, live, self_key, acc, msum, red, mred, [&](int e) { return ch + LPR * e; });
 }
 
 namespace {
@@ -413,7 +577,7 @@ bool fast_args(const DecodeParams& p, DecodeFastArgs* a) {
 
 }  // namespace
 
-int launch_decode(int flow, bool f64, const DecodeParams& p_in, hipStream_t st, hipError_t* err) {
+int launch_decode(int flow, int rows, bool f64, const DecodeParams& p_in, hipStream_t st, hipError_t* err) {
   DecodeFastArgs p;
   bool fast = flow != DECODE_EXACT && !(flow == DECODE_F32 && p_in.W > 512);
   if (fast && !fast_args(p_in, &p)) fast = false;
@@ -483,11 +647,23 @@ int launch_decode(int flow, bool f64, const DecodeParams& p_in, hipStream_t st, 
     else DECODE_FAST(false);
 #undef DECODE_FAST
   } else {
-    const unsigned grid = (unsigned)((p_in.N * p_in.H + 63) / 64);
-    if (f64)
-      hipLaunchKernelGGL(decode_exact<double>, dim3(grid), dim3(64), 0, st, p_in);
-    else
-      hipLaunchKernelGGL(decode_exact<float>, dim3(grid), dim3(64), 0, st, p_in);
+    const dim3 grid((unsigned)(p_in.N * p_in.H));
+#define DECODE_ROWS(QT, VT)                                                                       \
+  do {                                                                                            \
+    if (p_in.D == 32)                                                                             \
+      hipLaunchKernelGGL((decode_rows<QT, VT, 4>), grid, dim3(64 * kRowsNW), 0, st, p_in);        \
+    else if (p_in.D == 64)                                                                        \
+      hipLaunchKernelGGL((decode_rows<QT, VT, 8>), grid, dim3(64 * kRowsNW), 0, st, p_in);        \
+    else                                                                                          \
+      hipLaunchKernelGGL((decode_rows<QT, VT, 16>), grid, dim3(64 * kRowsNW), 0, st, p_in);       \
+  } while (0)
+    if (rows == DECODE_BF16) DECODE_ROWS(bf16, bf16);
+    else if (rows == DECODE_F16) DECODE_ROWS(f16, f16);
+    else if (rows == DECODE_KF32) DECODE_ROWS(float, bf16);
+    else if (rows == DECODE_F32) DECODE_ROWS(float, float);
+    else if (f64) hipLaunchKernelGGL(decode_any<double>, grid, dim3(256), 0, st, p_in);
+    else hipLaunchKernelGGL(decode_any<float>, grid, dim3(256), 0, st, p_in);
+#undef DECODE_ROWS
   }
   *err = hipGetLastError();
   return 0;
