@@ -60,20 +60,33 @@ __device__ __forceinline__ void f16x8_to_f32(const u16x8& u, float* x) {
 
 // ----------------------------------------------------------------- terms
 
-// 8 float32 values -> NT bf16 bit patterns per value.
+// 8 float32 values -> NT bf16 bit patterns per value, two values to each
+// packed conversion: a term of a pair comes back to float32 by one shift and
+// one mask of the packed word, 11 VALU instructions per pair for NT = 3 (taken
+// value by value the compiler made one conversion per value and term and
+// packed the halves afterwards: 16 to 17).  At B8 H16 T1024 d64 W256, autocast
+// types: 266.6 -> 255.6 us per fwd+bwd, results bit for bit the same.
 template <int NT>
 __device__ __forceinline__ void split8(const float* x, u16x8* t) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  u32x4 u[NT];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const bf16 h = (bf16)x[e];
-    t[0][e] = bf16_bits(h);
-    if constexpr (NT >= 2) {
-      const float r = x[e] - (float)h;
-      const bf16 m = (bf16)r;
-      t[1][e] = bf16_bits(m);
-      if constexpr (NT == 3) t[2][e] = bf16_bits((bf16)(r - (float)m));
+  for (int e = 0; e < 4; ++e) {
+    f32x2 v = {x[2 * e], x[2 * e + 1]};
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+      u[i][e] = w;
+      if (i + 1 < NT) {
+        v[0] -= __builtin_bit_cast(float, w << 16);
+        v[1] -= __builtin_bit_cast(float, w & 0xffff0000u);
+      }
     }
   }
+#pragma unroll
+  for (int i = 0; i < NT; ++i) t[i] = __builtin_bit_cast(u16x8, u[i]);
 }
 
 // C += sum of A_i B_j over i < NA, j < NB, i + j <= L, largest i + j first.
