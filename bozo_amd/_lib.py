@@ -8,12 +8,14 @@ device pointers are valid inside it.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 
 import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libtension_hip.so")
+HOST_PATH = os.path.join(_HERE, "lib", "_host.so")
 
 # dtype codes (enum in tension_hip.h)
 F32, BF16, F16, F64 = 0, 1, 2, 3
@@ -97,6 +99,23 @@ def lib():
             fn.argtypes = args
         _lib = h
     return _lib
+
+
+_host = None
+
+
+def host():
+    """Load (once) and return the native call path (csrc/host.cpp)."""
+    global _host
+    if _host is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise TensionError(f"{HOST_PATH} is missing: build it with `python -m bozo_amd.build`")
+        spec = importlib.util.spec_from_file_location("bozo_amd._host", HOST_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        _host = mod
+    return _host
 
 
 def check(status: int, what: str) -> None:

@@ -3,7 +3,9 @@
     python -m bozo_amd.build          # always recompiles
 
 Each HIP translation unit is compiled in parallel to an object file under
-bozo_amd/_build/, then linked into bozo_amd/lib/libtension_hip.so.
+bozo_amd/_build/, then linked into bozo_amd/lib/libtension_hip.so.  The eager
+call path (csrc/host.cpp, host code only) is compiled with the C++ compiler
+against the installed torch and linked to that library: bozo_amd/lib/_host.so.
 """
 from __future__ import annotations
 
@@ -12,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -20,6 +23,7 @@ INCLUDE = os.path.join(ROOT, "include")
 OBJDIR = os.path.join(PKG, "_build")
 LIBDIR = os.path.join(PKG, "lib")
 LIBNAME = "libtension_hip.so"
+HOSTNAME = "_host.so"
 ARCH = os.environ.get("TENSION_OFFLOAD_ARCH", "gfx950")
 
 SOURCES = [
@@ -65,11 +69,40 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _host_compile() -> str:
+    import torch
+    from torch.utils import cpp_extension
+    obj = os.path.join(OBJDIR, "host.o")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall",
+           "-DTORCH_EXTENSION_NAME=_host", "-DTORCH_API_INCLUDE_EXTENSION_H", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE]
+    for d in [*cpp_extension.include_paths("cuda"), sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", d]
+    r = subprocess.run(cmd + ["-c", os.path.join(CSRC, "host.cpp"), "-o", obj], capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on host.cpp:\n{r.stdout}\n{r.stderr}")
+    return obj
+
+
+def _host_link(obj: str) -> None:
+    from torch.utils import cpp_extension
+    out = os.path.join(LIBDIR, HOSTNAME)
+    cmd = [os.environ.get("CXX", "g++"), "-shared", obj, "-o", out + ".tmp",
+           *[f"-L{d}" for d in cpp_extension.library_paths("cuda")], "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch",
+           "-ltorch_python", f"-L{LIBDIR}", f"-l:{LIBNAME}", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"link of {HOSTNAME} failed:\n{r.stdout}\n{r.stderr}")
+    os.replace(out + ".tmp", out)
+
+
 def build(verbose: bool = True) -> str:
     os.makedirs(OBJDIR, exist_ok=True)
     os.makedirs(LIBDIR, exist_ok=True)
     with cf.ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 4, 16)) as ex:
+        host = ex.submit(_host_compile)
         objs = list(ex.map(_compile, SOURCES))
+        host_obj = host.result()
     out = os.path.join(LIBDIR, LIBNAME)
     tmp = out + ".tmp"
     cmd = [hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp]
@@ -77,6 +110,7 @@ def build(verbose: bool = True) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, out)
+    _host_link(host_obj)
     if verbose:
         print(f"built {out}")
     return out

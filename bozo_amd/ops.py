@@ -62,28 +62,12 @@ def _rows(t: Optional[Tensor]) -> Optional[Tensor]:
     return t
 
 
-def _acc_code(*ts: Tensor) -> int:
-    return L.F64 if any(t.dtype == torch.float64 for t in ts) else L.F32
-
-
 def _side(t: Optional[Tensor], like: Tensor) -> Optional[Tensor]:
     """Side inputs (bias) are kept in float32, as the reference does
     (ops.py:93), or float64 for float64 calls."""
     if t is None:
         return None
     return _rows(t.to(torch.float64 if like.dtype == torch.float64 else torch.float32))
-
-
-def _stream(t: Tensor):
-    return L.stream_handle(t.device)
-
-
-def _ws(nbytes: int, dev) -> Optional[Tensor]:
-    return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes > 0 else None
-
-
-def _ptr(t: Optional[Tensor]):
-    return None if t is None else t.data_ptr()
 
 
 def _grads_like(*ts: Tensor):
@@ -117,15 +101,24 @@ def _note_exact_path(what: str, Q: Tensor, K: Tensor, V: Tensor, pairs: int) -> 
                   stacklevel=3)
 
 
-def _window_fwd(Q, K, V, W, scale, tau, bias, flags, mass):
-    B, T, H, D = Q.shape
-    out = torch.empty(B, T, H, D, dtype=Q.dtype, device=Q.device)
-    with torch.cuda.device(Q.device):
-        L.check(L.lib().tension_window_fwd(
-            L.buf(Q), L.buf(K), L.buf(V), L.buf(out), L.buf(tau), L.buf(bias), L.buf(mass),
-            B, T, H, D, W, float(scale), flags, _stream(Q)), "tension_window_fwd")
-    _note_exact_path("causal_tension", Q, K, V, B * T * H * min(int(W), T))
-    return out
+def _eager() -> bool:
+    """The native autograd nodes (csrc/host.cpp) run the call: not while
+    torch.jit traces (which records the Python Functions below) or inside a
+    functorch transform (which refuses them)."""
+    return torch._C._get_tracing_state() is None and not torch._C._are_functorch_transforms_active()
+
+
+def _supported(*ts: Optional[Tensor]) -> None:
+    for t in ts:
+        if t is not None and t.dtype not in L.DTYPE_CODE:
+            raise TypeError(f"unsupported dtype {t.dtype}")
+
+
+def _window_fwd(Q, K, V, W, scale, return_tau, bias, flags, want_mass):
+    """out, tau (None unless asked for), tau mass (likewise)."""
+    res = L.host().window_fwd(Q, K, V, bias, int(W), float(scale), flags, return_tau, want_mass)
+    _note_exact_path("causal_tension", Q, K, V, Q.shape[0] * Q.shape[1] * Q.shape[2] * min(int(W), Q.shape[1]))
+    return res
 
 
 class _CausalTensionFn(torch.autograd.Function):
@@ -133,19 +126,14 @@ class _CausalTensionFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, Q, K, V, W: int, scale: float, return_tau: bool, bias, normalize=None):
-        B, T, H, D = Q.shape
         flags = _NORMS[normalize]
         Bias = _side(bias, Q)
-        if Bias is not None and tuple(Bias.shape) != (B, T, W):
-            raise ValueError(f"bias must be [B, T, W]=[{B}, {T}, {W}], got {tuple(Bias.shape)}")
-        tau = torch.empty(B, T, H, W, dtype=Q.dtype, device=Q.device) if return_tau else None
         # the backward recomputes tau from the inputs; with float32 Q / K
         # under tau-mass it takes the per-query coefficients from the
         # forward's float32 rows and tau mass where that is the faster dQ
         # (tension_window_bwd_saved: one pass over the band instead of two)
-        rows = _saved_rows_flow(Q, K, V, W, flags)
-        mass = torch.empty(B, T, H, dtype=torch.float32, device=Q.device) if rows else None
-        out = _window_fwd(Q, K, V, W, scale, tau, Bias, flags, mass)
+        rows = L.host().saved_rows_flow(Q, K, V, W, flags)
+        out, tau, mass = _window_fwd(Q, K, V, W, scale, return_tau, Bias, flags, rows)
         if rows:
             ctx.save_for_backward(Q, K, V, Bias, out, mass)
         else:
@@ -168,39 +156,8 @@ class _CausalTensionFn(torch.autograd.Function):
         return dQ, dK, dV, None, None, None, None, None
 
 
-def _saved_rows_flow(Q: Tensor, K: Tensor, V: Tensor, W: int, flags: int) -> bool:
-    """Tau-mass with float32 Q / K at head dim 32 / 64, where the backward
-    takes its coefficients from the forward's rows: with a bf16 V (the
-    reference's autocast flow) for windows wider than 64 (narrower bands
-    form them in registers, which is faster), with a float32 V at every
-    window (its dQ kernel keeps no band in registers)."""
-    if not (flags & L.NORM_MASS) or Q.dtype != torch.float32 or K.dtype != torch.float32 \
-            or Q.shape[-1] not in (32, 64):
-        return False
-    if V.dtype == torch.bfloat16:
-        return W > 64
-    return V.dtype == torch.float32
-
-
 def _window_bwd(Q, K, V, dOut, dTau, Bias, W, scale, flags, out=None, mass=None):
-    B, T, H, D = Q.shape
-    dOut = _rows(dOut) if dOut is not None else torch.zeros_like(Q)
-    dTau = _rows(dTau)
-    dQ, dK, dV = _grads_like(Q, K, V)
-    lib = L.lib()
-    ws = _ws(lib.tension_window_bwd_workspace(B, T, H, _acc_code(Q, K, V), flags), Q.device)
-    with torch.cuda.device(Q.device):
-        if out is not None:
-            L.check(lib.tension_window_bwd_saved(
-                L.buf(Q), L.buf(K), L.buf(V), L.buf(dOut), L.buf(dTau), L.buf(Bias), L.buf(out),
-                L.buf(mass), L.buf(dQ), L.buf(dK), L.buf(dV), _ptr(ws), B, T, H, D, W,
-                float(scale), flags, _stream(Q)), "tension_window_bwd_saved")
-        else:
-            L.check(lib.tension_window_bwd(
-                L.buf(Q), L.buf(K), L.buf(V), L.buf(dOut), L.buf(dTau), L.buf(Bias),
-                L.buf(dQ), L.buf(dK), L.buf(dV), _ptr(ws), B, T, H, D, W,
-                float(scale), flags, _stream(Q)), "tension_window_bwd")
-    return dQ, dK, dV
+    return L.host().window_bwd(Q, K, V, dOut, dTau, Bias, out, mass, int(W), float(scale), flags)
 
 
 def causal_tension(Q: Tensor, K: Tensor, V: Tensor, window: int, scale: float,
@@ -234,8 +191,16 @@ def causal_tension(Q: Tensor, K: Tensor, V: Tensor, window: int, scale: float,
         out, tau = torch.ops.bozo.window_fwd(Q, K, V, int(window), float(scale), bool(return_tau), Bias,
                                              _NORMS[normalize])
         return (out, tau) if return_tau else out
-    return _CausalTensionFn.apply(_rows(Q), _rows(K), _rows(V), int(window), float(scale),
-                                  bool(return_tau), bias, normalize)
+    _supported(Q, K, V)
+    B, T, H, _ = Q.shape
+    W = int(window)
+    if bias is not None and tuple(bias.shape) != (B, T, W):
+        raise ValueError(f"bias must be [B, T, W]=[{B}, {T}, {W}], got {tuple(bias.shape)}")
+    if not _eager():
+        return _CausalTensionFn.apply(_rows(Q), _rows(K), _rows(V), W, float(scale), bool(return_tau), bias, normalize)
+    res = L.host().window(Q, K, V, bias, W, float(scale), _NORMS[normalize], bool(return_tau))
+    _note_exact_path("causal_tension", Q, K, V, B * T * H * min(W, T))
+    return (res[0], res[1]) if return_tau else res[0]
 
 
 # ----------------------------------------------------------------- global block
@@ -246,11 +211,8 @@ class _GlobalTensionFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, Q, K, V, scale: float, bias, W_local):
-        B, T, H, D = Q.shape
         Bias = _side(bias, Q)
-        if Bias is not None and tuple(Bias.shape) != (B, T, T):
-            raise ValueError(f"global bias must be [B, T, T]=[{B}, {T}, {T}], got {tuple(Bias.shape)}")
-        Wl = 0 if W_local is None else min(int(W_local), T)
+        Wl = 0 if W_local is None else min(int(W_local), Q.shape[1])
         out, tl, mass = _global_fwd(Q, K, V, scale, Bias, Wl)
         ctx.save_for_backward(Q, K, V, Bias, out, mass)
         ctx.scale, ctx.Wl = scale, Wl
@@ -268,33 +230,14 @@ class _GlobalTensionFn(torch.autograd.Function):
 
 def _global_fwd(Q, K, V, scale, Bias, Wl):
     """out, tau_local (None when Wl is 0) and the tau mass of the global block."""
-    B, T, H, D = Q.shape
-    tl = torch.empty(B, T, H, Wl, dtype=Q.dtype, device=Q.device) if Wl > 0 else None
-    out = torch.empty_like(Q)
-    # the tau mass per query, kept with the output so the backward gets
-    # its per-query coefficients from these rows (no band recompute)
-    mass = torch.empty(B, T, H, dtype=torch.float32, device=Q.device)
-    with torch.cuda.device(Q.device):
-        L.check(L.lib().tension_global_fwd(
-            L.buf(Q), L.buf(K), L.buf(V), L.buf(out), L.buf(tl), L.buf(Bias), L.buf(mass),
-            B, T, H, D, Wl, float(scale), 0, _stream(Q)), "tension_global_fwd")
+    B, T, H, _ = Q.shape
+    res = L.host().global_fwd(Q, K, V, Bias, float(scale), Wl)
     _note_exact_path("global_tension", Q, K, V, B * H * T * (T + 1) // 2)
-    return out, tl, mass
+    return res
 
 
 def _global_bwd(Q, K, V, dOut, dTl, Bias, out, mass, Wl, scale):
-    B, T, H, D = Q.shape
-    dOut = _rows(dOut) if dOut is not None else torch.zeros_like(Q)
-    dTl = _rows(dTl) if Wl > 0 else None
-    dQ, dK, dV = _grads_like(Q, K, V)
-    lib = L.lib()
-    ws = _ws(lib.tension_global_bwd_workspace(B, T, H, _acc_code(Q, K, V), 0), Q.device)
-    with torch.cuda.device(Q.device):
-        L.check(lib.tension_global_bwd(
-            L.buf(Q), L.buf(K), L.buf(V), L.buf(dOut), L.buf(dTl), L.buf(Bias), L.buf(out),
-            L.buf(mass), L.buf(dQ), L.buf(dK), L.buf(dV), _ptr(ws), B, T, H, D, Wl,
-            float(scale), 0, _stream(Q)), "tension_global_bwd")
-    return dQ, dK, dV
+    return L.host().global_bwd(Q, K, V, dOut, dTl, Bias, out, mass, Wl, float(scale))
 
 
 def global_tension(Q: Tensor, K: Tensor, V: Tensor, scale: float,
@@ -309,15 +252,22 @@ def global_tension(Q: Tensor, K: Tensor, V: Tensor, scale: float,
     if Q.dim() != 4 or K.shape != Q.shape or V.shape != Q.shape:
         raise ValueError("Q, K, V must share one [B, T, H, HD] shape")
     _same_device(Q, K, V, bias)
+    B, T, H, _ = Q.shape
+    Wl = 0 if W_local is None else min(int(W_local), T)
     if torch.compiler.is_compiling():  # the registered op, which torch.compile traces through
-        B, T = Q.shape[:2]
         Bias = _side(bias, Q)
         if Bias is not None and tuple(Bias.shape) != (B, T, T):
             raise ValueError(f"global bias must be [B, T, T]=[{B}, {T}, {T}], got {tuple(Bias.shape)}")
-        Wl = 0 if W_local is None else min(int(W_local), T)
         out, tl, _ = torch.ops.bozo.global_fwd(Q, K, V, float(scale), Bias, Wl)
         return (out, tl) if Wl > 0 else out
-    return _GlobalTensionFn.apply(_rows(Q), _rows(K), _rows(V), float(scale), bias, W_local)
+    _supported(Q, K, V)
+    if bias is not None and tuple(bias.shape) != (B, T, T):
+        raise ValueError(f"global bias must be [B, T, T]=[{B}, {T}, {T}], got {tuple(bias.shape)}")
+    if not _eager():
+        return _GlobalTensionFn.apply(_rows(Q), _rows(K), _rows(V), float(scale), bias, W_local)
+    res = L.host().global_(Q, K, V, bias, float(scale), Wl)
+    _note_exact_path("global_tension", Q, K, V, B * H * T * (T + 1) // 2)
+    return (res[0], res[1]) if Wl > 0 else res[0]
 
 
 # ----------------------------------------------------------------- decode
@@ -360,20 +310,17 @@ def decode_step(q: Tensor, k_new: Tensor, v_new: Tensor, k_cache: Tensor, v_cach
     (number of keys) or False / None (raw sum).  ``include_self``: the new
     token is a key too (a global layer's step; no tau then).  Returns out
     [N,H,D] in q.dtype."""
+    flags = _DECODE_NORMS.get(normalize)
+    if flags is not None:
+        out = L.host().decode_step(q, k_new, v_new, k_cache, v_cache, pos_in, pos_out, float(scale),
+                                   flags | (L.DECODE_SELF if include_self else 0), tau)
+        if out is not None:
+            return out
+    # refused: say why
     _on_gpu(q, k_new, v_new, k_cache, v_cache, pos_in, pos_out, tau)
     _check_decode_operands(q, k_new, v_new, k_cache, v_cache, pos_in, pos_out, tau)
-    N, H, D = q.shape
-    W = k_cache.shape[2]
-    if normalize not in _DECODE_NORMS:
-        raise ValueError(f"normalize must be one of {list(_DECODE_NORMS)}")
-    flags = _DECODE_NORMS[normalize] | (L.DECODE_SELF if include_self else 0)
-    out = torch.empty_like(q)
-    with torch.cuda.device(q.device):
-        L.check(L.lib().tension_decode_step(
-            L.buf(_rows(q)), L.buf(_rows(k_new)), L.buf(_rows(v_new)), L.buf(k_cache), L.buf(v_cache),
-            L.buf(out), L.buf(tau), pos_in.data_ptr(), _ptr(pos_out), N, H, D, W, float(scale),
-            flags, _stream(q)), "tension_decode_step")
-    return out
+    _supported(q, k_new, v_new, k_cache, v_cache, tau)
+    raise ValueError(f"normalize must be one of {list(_DECODE_NORMS)}")
 
 
 class TensionDecodeCache:
@@ -414,29 +361,21 @@ def autocast_inputs(*ts: Tensor):
 
 # ----------------------------------------------------------------- RoPE
 
-def _rope_call(x: Tensor, y: Tensor, cos: Tensor, sin: Tensor, pos_offset: int, inverse: int):
-    B, T, H, D = x.shape
-    with torch.cuda.device(x.device):
-        L.check(L.lib().tension_rope(L.buf(x), L.buf(y), cos.data_ptr(), sin.data_ptr(), cos.shape[0],
-                                     B, T, H, D, pos_offset, inverse, _stream(x)), "tension_rope")
+def _rope_call(x: Tensor, cos: Tensor, sin: Tensor, pos_offset: int, out_dtype: torch.dtype, inverse: int) -> Tensor:
+    return L.host().rope_call(x, cos, sin, int(pos_offset), out_dtype, inverse)
 
 
 class _RopeFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, cos, sin, pos_offset, out_dtype):
-        y = torch.empty(x.shape, dtype=out_dtype or x.dtype, device=x.device)
-        _rope_call(x, y, cos, sin, pos_offset, 0)
         ctx.save_for_backward(cos, sin)
         ctx.pos_offset, ctx.in_dtype = pos_offset, x.dtype
-        return y
+        return _rope_call(x, cos, sin, pos_offset, out_dtype or x.dtype, 0)
 
     @staticmethod
     def backward(ctx, dy):
         cos, sin = ctx.saved_tensors
-        dy = _rows(dy)
-        dx = torch.empty(dy.shape, dtype=ctx.in_dtype, device=dy.device)
-        _rope_call(dy, dx, cos, sin, ctx.pos_offset, 1)
-        return dx, None, None, None, None
+        return _rope_call(_rows(dy), cos, sin, ctx.pos_offset, ctx.in_dtype, 1), None, None, None, None
 
 
 def rope(x: Tensor, cos: Tensor, sin: Tensor, pos_offset: int = 0,
@@ -457,7 +396,10 @@ def rope(x: Tensor, cos: Tensor, sin: Tensor, pos_offset: int = 0,
     if torch.compiler.is_compiling():  # the registered op, which torch.compile traces through
         return torch.ops.bozo.rope(x, cos.contiguous(), sin.contiguous(), int(pos_offset),
                                    out_dtype or x.dtype, 0)
-    return _RopeFn.apply(_rows(x), cos.contiguous(), sin.contiguous(), int(pos_offset), out_dtype)
+    _supported(x)
+    if not _eager():
+        return _RopeFn.apply(_rows(x), cos.contiguous(), sin.contiguous(), int(pos_offset), out_dtype)
+    return L.host().rope(x, cos, sin, int(pos_offset), out_dtype)
 
 
 # ----------------------------------------------------------------- torch.library registration
@@ -475,10 +417,8 @@ def _op_window_fwd(Q: Tensor, K: Tensor, V: Tensor, window: int, scale: float, r
     B, T, H, _ = Q.shape
     if bias is not None and tuple(bias.shape) != (B, T, window):
         raise ValueError(f"bias must be [B, T, W]=[{B}, {T}, {window}], got {tuple(bias.shape)}")
-    Q, K, V = _rows(Q), _rows(K), _rows(V)
-    tau = torch.empty(B, T, H, window, dtype=Q.dtype, device=Q.device) if return_tau else Q.new_empty(0)
-    out = _window_fwd(Q, K, V, window, scale, tau if return_tau else None, bias, flags, None)
-    return out, tau
+    out, tau, _ = _window_fwd(_rows(Q), _rows(K), _rows(V), window, scale, return_tau, bias, flags, False)
+    return out, (tau if tau is not None else Q.new_empty(0))
 
 
 @_op_window_fwd.register_fake
@@ -562,10 +502,7 @@ _op_global_fwd.register_autograd(_global_grad, setup_context=_global_setup)
 @torch.library.custom_op("bozo::rope", mutates_args=(), device_types="cuda")
 def _op_rope(x: Tensor, cos: Tensor, sin: Tensor, pos_offset: int, out_dtype: torch.dtype,
              inverse: int) -> Tensor:
-    x = _rows(x)
-    y = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    _rope_call(x, y, cos, sin, pos_offset, inverse)
-    return y
+    return _rope_call(_rows(x), cos, sin, pos_offset, out_dtype, inverse)
 
 
 @_op_rope.register_fake
