@@ -341,9 +341,19 @@ __global__ __launch_bounds__(64 * NW) void decode_d64(DecodeFastArgs p) {
 // fast path.  libm exp and IEEE division, sums in A.  N16 H12 D64, 700 of
 // 1024 slots live, float32 self-key: 17.4 ms with one thread per (n, h).
 
-// One wave's row dot product over LPR lanes (a power of two, at most 64).
-template <int LPR, typename A>
-__device__ __forceinline__ A lanes_sum(A x) {
+// Sum over an aligned group of LPR lanes (4, 8 or 16, all active); in float
+// through DPP moves, whose latency is a VALU instruction's and not an LDS
+// round trip's.
+template <int LPR>
+__device__ __forceinline__ float lanes_sum(float x) {
+  x += dpp_move<0xB1>(x);  // lane ^ 1
+  x += dpp_move<0x4E>(x);  // lane ^ 2
+  if constexpr (LPR >= 8) x += dpp_move<0x141>(x);   // row_half_mirror: i <-> 7 - i
+  if constexpr (LPR >= 16) x += dpp_move<0x140>(x);  // row_mirror: i <-> 15 - i
+  return x;
+}
+template <int LPR>
+__device__ __forceinline__ double lanes_sum(double x) {
 #pragma unroll
   for (int m = 1; m < LPR; m <<= 1) x += __shfl_xor(x, m);
   return x;
@@ -394,19 +404,25 @@ __device__ __forceinline__ void decode_finish(const DecodeParams& p, int n, int 
   if (tid == 0 && h == 0 && p.pos_out) p.pos_out[n] = pos + 1;
 }
 
-// 16-byte aligned rows of 8 LPR elements: a lane holds 8 consecutive features
-// and keeps U rows of K and V in flight ahead of the U it works on.  QT: q,
-// k_new, the K cache and out; VT: v_new and the V cache.
+// 16-byte aligned rows of 8 LPR elements.  A lane's 8 features of a row: chunk
+// ch of a 16-bit row, chunks ch and LPR + ch of a float32 one, so every load
+// instruction covers whole contiguous row pieces.  QT: q, k_new, the K cache and
+// out; VT: v_new and the V cache.
 template <typename T>
 struct Row8 {
-  u16x8 a, b;  // b: the second half of a float32 row piece
+  u16x8 a, b;  // b: a float32 row's second chunk
 };
 
-template <typename T>
-__device__ __forceinline__ Row8<T> row8_load(const T* p) {
+template <int LPR, typename T>
+__device__ __forceinline__ int row8_feat(int ch, int e) {
+  return sizeof(T) == 2 ? 8 * ch + e : e < 4 ? 4 * ch + e : 4 * (LPR + ch) + e - 4;
+}
+
+template <int LPR, typename T>
+__device__ __forceinline__ Row8<T> row8_load(const T* row, int ch) {
   Row8<T> r;
-  r.a = __builtin_nontemporal_load((const u16x8*)p);
-  if constexpr (sizeof(T) == 4) r.b = __builtin_nontemporal_load((const u16x8*)(p + 4));
+  r.a = __builtin_nontemporal_load((const u16x8*)(row + row8_feat<LPR, T>(ch, 0)));
+  if constexpr (sizeof(T) == 4) r.b = __builtin_nontemporal_load((const u16x8*)(row + row8_feat<LPR, T>(ch, 4)));
   return r;
 }
 
@@ -430,11 +446,13 @@ __device__ __forceinline__ void row8_f32(const Row8<T>& r, float* x) {
   }
 }
 
-constexpr int kRowsNW = 8;  // waves per workgroup of decode_rows
+// Waves per workgroup: 4, or 16 for a long cache on a grid that would leave most
+// wave slots empty (kRowsU rows of K and V per lane in flight either way).
+constexpr int kRowsU = 4;
 
-template <typename QT, typename VT, int LPR>
-__global__ __launch_bounds__(64 * kRowsNW) void decode_rows(DecodeParams p) {
-  constexpr int NW = kRowsNW, U = 4, RPW = 64 / LPR;
+template <typename QT, typename VT, int LPR, int NW>
+__global__ __launch_bounds__(64 * NW) void decode_rows(DecodeParams p) {
+  constexpr int U = kRowsU, RPW = 64 / LPR;
   __shared__ float red[NW * 8 * LPR], mred[NW];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int ch = lane % LPR;
@@ -445,19 +463,9 @@ __global__ __launch_bounds__(64 * kRowsNW) void decode_rows(DecodeParams p) {
   const bool self_key = (p.flags & TENSION_DECODE_SELF) != 0;
   const float scale = (float)p.scale;
   float q[8];
-  row8_f32(row8_load((const QT*)p.q.p + n * p.q.s0 + h * p.q.s1 + 8 * ch), q);
-  const QT* kb = (const QT*)p.kc.p + n * p.kc.s0 + h * p.kc.s1 + 8 * ch;
-  const VT* vb = (const VT*)p.vc.p + n * p.vc.s0 + h * p.vc.s1 + 8 * ch;
-  // rows s0 + u RPW NW of one trip (past the cache: its last row, unused)
-  auto load = [&](int s0, Row8<QT>* k, Row8<VT>* v) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u * RPW * NW;
-      const int64_t r = s < W ? s : W - 1;
-      k[u] = row8_load(kb + r * p.kc.s2);
-      v[u] = row8_load(vb + r * p.vc.s2);
-    }
-  };
+  row8_f32(row8_load<LPR>((const QT*)p.q.p + n * p.q.s0 + h * p.q.s1, ch), q);
+  const QT* kb = (const QT*)p.kc.p + n * p.kc.s0 + h * p.kc.s1;
+  const VT* vb = (const VT*)p.vc.p + n * p.vc.s0 + h * p.vc.s1;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0}, msum = 0.f;
   auto tau_of = [&](const Row8<QT>& k) __attribute__((always_inline)) {
     float x[8], dot = 0.f;
@@ -473,13 +481,21 @@ __global__ __launch_bounds__(64 * kRowsNW) void decode_rows(DecodeParams p) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] += tau * x[e];
   };
-  const int first = wave * RPW + lane / LPR, trip = RPW * NW * U;
-  Row8<QT> k[U], kn[U];
-  Row8<VT> v[U], vn[U];
-  if (rows > 0) load(first, k, v);
-  for (int base = 0; base < rows; base += trip) {
-    const bool more = base + trip < rows;
-    if (more) load(base + trip + first, kn, vn);
+  const int first = wave * RPW + lane / LPR;
+  for (int base = 0; base < rows; base += RPW * NW * U) {
+    Row8<QT> k[U];
+    Row8<VT> v[U];
+    // past the cache: its last row, unused
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = base + first + u * RPW * NW;
+      k[u] = row8_load<LPR>(kb + (int64_t)(s < W ? s : W - 1) * p.kc.s2, ch);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = base + first + u * RPW * NW;
+      v[u] = row8_load<LPR>(vb + (int64_t)(s < W ? s : W - 1) * p.vc.s2, ch);
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int s = base + first + u * RPW * NW;
@@ -489,20 +505,14 @@ __global__ __launch_bounds__(64 * kRowsNW) void decode_rows(DecodeParams p) {
       if (p.tau.p && ch == 0 && s < W)
         st<float>(p.tau, n * p.tau.s0 + h * p.tau.s1 + ring_w(s, pos, W), s < live ? t : 0.f);
     }
-    if (more) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        k[u] = kn[u];
-        v[u] = vn[u];
-      }
-    }
   }
   if (self_key && wave == 0) {  // the new token as a key: row group 0 of wave 0
-    const float t = tau_of(row8_load((const QT*)p.kn.p + n * p.kn.s0 + h * p.kn.s1 + 8 * ch));
-    const Row8<VT> sv = row8_load((const VT*)p.vn.p + n * p.vn.s0 + h * p.vn.s1 + 8 * ch);
+    const float t = tau_of(row8_load<LPR>((const QT*)p.kn.p + n * p.kn.s0 + h * p.kn.s1, ch));
+    const Row8<VT> sv = row8_load<LPR>((const VT*)p.vn.p + n * p.vn.s0 + h * p.vn.s1, ch);
     if (lane < LPR) add(t, sv);
   }
-  decode_finish<LPR, NW, 8>(p, n, h, pos, live, self_key, acc, msum, red, mred, [&](int e) { return 8 * ch + e; });
+  decode_finish<LPR, NW, 8>(p, n, h, pos, live, self_key, acc, msum, red, mred,
+                            [&](int e) { return row8_feat<LPR, VT>(ch, e); });
 }
 
 // Any dtypes, alignment and D <= 256: 16 lanes per row, lane l holds features
@@ -648,14 +658,19 @@ int launch_decode(int flow, int rows, bool f64, const DecodeParams& p_in, hipStr
 #undef DECODE_FAST
   } else {
     const dim3 grid((unsigned)(p_in.N * p_in.H));
-#define DECODE_ROWS(QT, VT)                                                                       \
-  do {                                                                                            \
-    if (p_in.D == 32)                                                                             \
-      hipLaunchKernelGGL((decode_rows<QT, VT, 4>), grid, dim3(64 * kRowsNW), 0, st, p_in);        \
-    else if (p_in.D == 64)                                                                        \
-      hipLaunchKernelGGL((decode_rows<QT, VT, 8>), grid, dim3(64 * kRowsNW), 0, st, p_in);        \
-    else                                                                                          \
-      hipLaunchKernelGGL((decode_rows<QT, VT, 16>), grid, dim3(64 * kRowsNW), 0, st, p_in);       \
+    // 16 waves where fewer than two workgroups per CU each have more than one
+    // 4-wave trip (64 / LPR x 4 x kRowsU rows) to make
+    const bool deep = (int64_t)p_in.N * p_in.H < 2 * device_cus() && (int64_t)p_in.W * p_in.D > 8 * 64 * 4 * kRowsU;
+#define DECODE_ROWS_D(QT, VT, LPR)                                                              \
+  do {                                                                                          \
+    if (deep) hipLaunchKernelGGL((decode_rows<QT, VT, LPR, 16>), grid, dim3(1024), 0, st, p_in); \
+    else hipLaunchKernelGGL((decode_rows<QT, VT, LPR, 4>), grid, dim3(256), 0, st, p_in);        \
+  } while (0)
+#define DECODE_ROWS(QT, VT)                       \
+  do {                                            \
+    if (p_in.D == 32) DECODE_ROWS_D(QT, VT, 4);   \
+    else if (p_in.D == 64) DECODE_ROWS_D(QT, VT, 8); \
+    else DECODE_ROWS_D(QT, VT, 16);               \
   } while (0)
     if (rows == DECODE_BF16) DECODE_ROWS(bf16, bf16);
     else if (rows == DECODE_F16) DECODE_ROWS(f16, f16);
@@ -664,6 +679,7 @@ int launch_decode(int flow, int rows, bool f64, const DecodeParams& p_in, hipStr
     else if (f64) hipLaunchKernelGGL(decode_any<double>, grid, dim3(256), 0, st, p_in);
     else hipLaunchKernelGGL(decode_any<float>, grid, dim3(256), 0, st, p_in);
 #undef DECODE_ROWS
+#undef DECODE_ROWS_D
   }
   *err = hipGetLastError();
   return 0;

@@ -1,7 +1,7 @@
 """Decode steps outside the head-dim-64 fast kernel, against the float64
 oracle: the row kernel (aligned rows of 32, 64 and 128 elements) around the
-edges of its trips -- 128, 256 and 512 rows at head dims 128, 64 and 32 --
-and the general one (other head dims, mixed dtypes, unaligned rows).  Dead
+edges of its trips -- 256, 128 and 64 rows at head dims 32, 64 and 128 with 4
+waves, four times that with 16 (a long cache on a small grid) -- and the general one (other head dims, mixed dtypes, unaligned rows).  Dead
 slots hold NaN: they are nobody's rows and must not be read into a result.
 
 Tolerances: float32 sums of W products of the float32 inputs differ from
@@ -23,9 +23,12 @@ pytestmark = pytest.mark.gpu
 
 _F32, _BF16, _F16, _F64 = torch.float32, torch.bfloat16, torch.float16, torch.float64
 
-# q / K dtype, V dtype, D, W, positions, self key, tau, storage offset of every tensor's rows
+# q / K dtype, V dtype, D, W, positions, self key, tau, storage offset of every tensor's rows, heads
 CASES = [
-    (_F32, _F32, 64, 1024, (0, 1, 255, 256, 257, 1023), True, False, 0),
+    (_F32, _F32, 64, 1024, (0, 1, 511, 512, 513, 1023), True, False, 0),
+    (_F32, _F32, 64, 300, (127, 128, 129, 256), True, False, 0, 130),      # 4 waves, several trips
+    (_BF16, _BF16, 32, 600, (255, 256, 257, 700), False, True, 0, 130),
+    (_F32, _BF16, 128, 130, (63, 64, 65, 128, 131), False, True, 0, 110),
     (_F32, _F32, 64, 600, (0, 3, 511, 600, 601, 1500), False, True, 0),
     (_BF16, _BF16, 64, 1500, (0, 1, 256, 700, 1499, 2900), False, True, 0),
     (_BF16, _BF16, 64, 2048, (1, 1030, 2047), True, False, 0),
@@ -46,11 +49,11 @@ CASES = [
 
 @pytest.mark.parametrize("norm", ["mass", "count", "raw"])
 @pytest.mark.parametrize("case", CASES, ids=[f"{str(c[0])[6:]}-{str(c[1])[6:]}-D{c[2]}W{c[3]}"
-                                             f"{'-self' if c[5] else ''}{'-off' if c[7] else ''}" for c in CASES])
+                                             f"{'-self' if c[5] else ''}{'-off' if c[7] else ''}-H{(*c, 3)[8]}" for c in CASES])
 def test_decode_rows(dev, case, norm):
     from bozo_amd import decode_step
-    qd, vd, D, W, where, self_key, want_tau, off = case
-    N, H = len(where), 3
+    qd, vd, D, W, where, self_key, want_tau, off, H = (*case, 3)[:9]
+    N = len(where)
     g = torch.Generator().manual_seed(41 + W + D)
     print(f"[decode rows {case} {norm}]", flush=True)
 
