@@ -29,6 +29,7 @@ ARCH = os.environ.get("TENSION_OFFLOAD_ARCH", "gfx950")
 SOURCES = [
     "capi.hip", "exact.hip", "decode.hip",
     "mfma.hip", "mfma_fwd.hip", "mfma_dq.hip", "mfma_dkv.hip", "mfma_bwd_fused.hip", "mfma_global.hip",
+    "mfma_wide.hip",
     "split.hip", "split_fwd_bf16.hip", "split_dq_bf16.hip", "split_dkv_bf16.hip",
     "split_fwd_f32.hip", "split_dq_f32.hip", "split_dkv_f32.hip",
     "split_fwd_f32v.hip", "split_dq_f32v.hip", "split_dkv_f32v.hip",

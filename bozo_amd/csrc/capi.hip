@@ -176,20 +176,11 @@ bool split_dv_rows(int kind, const tension_buf* b) {
 // them as typed rows).
 bool split_side(int kind, const tension_buf* b) { return !b || b->dtype == split_qk_dtype(kind); }
 
-// Local windows wider than one 64-row tile run on the split kernels in bf16
-// too: 14-20% faster per fwd+bwd step than the dedicated band kernels'
-// W > 64 path (mfma_fwd / mfma_dq / mfma_dkv), measured at W = 100, 128,
-// 256, tau-mass and valid-count.  TENSION_WIDE_ON_BAND_KERNELS keeps them
-// on the band kernels (for A/B runs).
-bool wide_on_split(bool global, int64_t W) {
-#ifdef TENSION_WIDE_ON_BAND_KERNELS
-  (void)global;
-  (void)W;
-  return false;
-#else
-  return !global && W > 64;
-#endif
-}
+// bf16 local windows wider than one 64-row tile: without side operands (bias,
+// tau, dTau) on the wide band kernels (mfma_wide.hip); with them on the split
+// kernels.  Forward + backward at B8 H16 T1024 W256, valid count: 109 us there,
+// 117 us on the split kernels.
+bool wide_on_split(bool global, int64_t W, bool side) { return !global && W > 64 && side; }
 
 enum {
   KERNEL_EXACT = 0,
@@ -265,7 +256,8 @@ int band_fwd(const tension_buf* q, const tension_buf* k, const tension_buf* v, c
   p.out = make_buf(out); p.tau = make_buf(tau); p.bias = make_buf(bias); p.mass = make_buf(mass);
   bool mf = !(flags & TENSION_FORCE_EXACT) && sh.D == 64 && aligned_bf16_rows(q) && aligned_bf16_rows(k) &&
                   aligned_bf16_rows(v) && aligned_bf16_rows(out) && (!bias || bias->dtype == TENSION_F32);
-  if (wide_on_split(global, Wparam)) mf = false;
+  // (the wide kernels write the tau mass only where it normalises)
+  if (wide_on_split(global, Wparam, bias || tau || (mass && !(flags & TENSION_NORM_MASS)))) mf = false;
   const int sk = mf ? SPLIT_NONE : split_kind(q, k, v, bias, sh.D, flags);
   const bool sp = sk != SPLIT_NONE && split_rows(sk, out) && split_side(sk, tau);
   return run_band(0, sp ? split_kernel(sk) : mf ? KERNEL_MFMA : KERNEL_EXACT, any_f64(q, k, v), p, stream, what);
@@ -343,7 +335,7 @@ int band_bwd_dq(const tension_buf* q, const tension_buf* k, const tension_buf* v
   BandParams p = bwd_params(q, k, v, dout, dtau, bias, ws, sh, Wparam, scale, flags, global);
   p.dq = make_buf(dq);
   bool mf = mfma_ok_bwd(q, k, v, dout, bias, dq, nullptr, sh.D, flags);
-  if (wide_on_split(global, Wparam)) mf = false;
+  if (wide_on_split(global, Wparam, bias || dtau)) mf = false;
   const int sk = mf ? SPLIT_NONE : split_kind(q, k, v, bias, sh.D, flags);
   const bool sp = sk != SPLIT_NONE && split_rows(sk, dout) && split_rows(sk, dq) && split_side(sk, dtau);
   // the forward's saved output rows and tau mass (the tau-mass coefficients
@@ -380,7 +372,7 @@ int band_bwd_dkv(const tension_buf* q, const tension_buf* k, const tension_buf* 
   p.dk = make_buf(dk);
   p.dv = make_buf(dv);
   bool mf = mfma_ok_bwd(q, k, v, dout, bias, dk, dv, sh.D, flags);
-  if (wide_on_split(global, Wparam)) mf = false;
+  if (wide_on_split(global, Wparam, bias || dtau)) mf = false;
   const int sk = mf ? SPLIT_NONE : split_kind(q, k, v, bias, sh.D, flags);
   const bool sp = sk != SPLIT_NONE && split_rows(sk, dout) && split_rows(sk, dk) && split_dv_rows(sk, dv) &&
                   split_side(sk, dtau);

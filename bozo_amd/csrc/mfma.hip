@@ -10,6 +10,7 @@ void launch_mfma_fwd(const BandParams& p, hipStream_t st, unsigned nwg, int norm
 void launch_mfma_dq(const BandParams& p, hipStream_t st, unsigned nwg, int norm);
 void launch_mfma_dkv(const BandParams& p, hipStream_t st, unsigned nwg, int norm);
 void launch_mfma_bwd_fused(const BandParams& p, hipStream_t st, unsigned nwg, int norm);
+void launch_wide(int phase, const BandParams& p, hipStream_t st, unsigned nwg, int norm);
 
 // Workgroups the fused backward aims for per CU: two resident (76 KB of LDS
 // each).
@@ -62,6 +63,13 @@ int launch_mfma(int phase, const BandParams& p_in, hipStream_t st, hipError_t* e
     if (bh * runs > 0x7fffffff) return kGridTooLarge;
     p.chunk = (int)runs;
     launch_mfma_bwd_fused(p, st, (unsigned)(bh * runs), norm);
+    *err = hipGetLastError();
+    return 0;
+  }
+  // a local window wider than a tile: the host takes this route without bias,
+  // tau and dTau only
+  if (!p.glob && p.win > kTile && phase >= 0 && phase <= 2) {
+    launch_wide(phase, p, st, (unsigned)nwg, norm);
     *err = hipGetLastError();
     return 0;
   }
