@@ -35,7 +35,7 @@ int launch_split(int phase, int flow, const BandParams& p_in, hipStream_t st, hi
   // 272 registers, one wave per SIMD, and one tile per workgroup measured
   // faster: 134 against 142 us per float32 step at B8 H12 T1024 W64), dQ
   // for float32 Q / K with a bf16 V at head dim 32 without dTau (where its
-  // run kernel measured faster); 0: one tile per workgroup
+  // run kernel measured faster); 0: one tile per workgroup; -1: see below
   p.chunk = 0;
   const bool dq_runs = flow == SPLIT_FLOW_F32 && p.D == 32 && p.dtau.p == nullptr;
   const bool dkv_runs = !(flow == SPLIT_FLOW_F32V && p.D == 64);
@@ -50,6 +50,13 @@ int launch_split(int phase, int flow, const BandParams& p_in, hipStream_t st, hi
       nwg = bh * runs;
     }
   }
+  // a forward whose bands span more than two key blocks, on a grid of at most one
+  // workgroup per CU: two key groups per workgroup (p.chunk < 0, xb_fwd).  B1
+  // H16 T1024, autocast / float32: W256 14.5 -> 12.6 / 18.0 -> 15.9 us, with tau
+  // 20.2 -> 17.7 / 23.7 -> 20.1, global 36.6 -> 27.6 / 47.9 -> 36.8; past one per
+  // CU the larger workgroups no longer all fit at once (B2 H12 T1024 with tau
+  // 25.8 -> 31.8 / 30.4 -> 35.8)
+  if (phase == 0 && (p.glob || p.win > 64) && nwg <= device_cus()) p.chunk = -1;
   const unsigned n = (unsigned)nwg;
   typedef void (*Launch)(const BandParams&, hipStream_t, unsigned);
   static const Launch table[4][3] = {

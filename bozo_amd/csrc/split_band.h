@@ -406,13 +406,6 @@ __device__ __forceinline__ void stage_get4(const E* st, int c, int j, int g, flo
   }
 }
 
-// Column of key `key` in query row t's tau, or -1 outside its band / slots.
-__device__ __forceinline__ int band_tau_col(const BandParams& p, int t, int key) {
-  const int lo = t - p.win > 0 ? t - p.win : 0;
-  if (key < lo || key > t - 1 + p.diag) return -1;
-  return tau_col(p, t, key);
-}
-
 // The raw pre-sigmoid bias of a lane's 16 pairs of one key block (query tq,
 // row `brow` of the bias; keys kb0 + 16 j + 4 g + r): loaded together ahead
 // of the block's products, so the loads' latency runs under them (a pair off
@@ -432,27 +425,58 @@ __device__ __forceinline__ void bias_block(const BandParams& p, const float* bro
 }
 
 // Rows t0w .. t0w + 15 (the wave's queries) of a [B,T,H,Wtau] tau / dTau of
-// this (b, h): lane l moves key kb0 + l of each row.
+// this (b, h): lane l moves key kb0 + l of each row.  A row's start is a uniform
+// address; the lane's column is key - t + W (local), one less from row to row,
+// on the band while it lies in [0, W), or T - 1 - key (global), the same for
+// every row, for keys up to t.  (With a column and a 64-bit offset worked out per
+// row and element, and the row's LDS read and store in turn: 38.6 against 36.1 us
+// for xb_fwd_run at B8 H12 T1024 d64 W64, autocast types, 54.0 against 53.1 for
+// its xb_dq, and 24.2 against 22.4 for the prefill at xb_fwd.)
+struct TauCol {
+  int col, step;   // the lane's column in row t0w and its step per row
+  unsigned width;  // columns [0, width) exist
+  int key0;        // global: the first row (of the 16) that sees the lane's key
+};
+
+__device__ __forceinline__ TauCol tau_lane_col(const BandParams& p, int t0w, int kb0, int lane) {
+  const int key = kb0 + lane;
+  if (p.glob) return {p.T - 1 - key, 0, (unsigned)p.Wtau, key - t0w};
+  return {key - t0w + p.W, -1, (unsigned)p.W, -1};
+}
+
+__device__ __forceinline__ bool tau_row_on(const TauCol& c, int rr) {
+  return (unsigned)(c.col + rr * c.step) < c.width && rr >= c.key0;
+}
+
 template <typename E>
 __device__ __forceinline__ void tau_rows_store(const BandParams& p, E* base, const E* st, int t0w, int kb0,
                                                int lane) {
-#pragma unroll 4
-  for (int rr = 0; rr < 16; ++rr) {
-    const int t = t0w + rr;
-    if (t >= p.T) break;
-    const int col = band_tau_col(p, t, kb0 + lane);
-    if (col >= 0) base[(int64_t)t * p.tau.s1 + col] = st[stage_at(rr, lane)];
+  const TauCol c = tau_lane_col(p, t0w, kb0, lane);
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    E v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = st[stage_at(8 * half + i, lane)];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int rr = 8 * half + i;
+      E* row = base + (int64_t)(t0w + rr) * p.tau.s1;
+      if (t0w + rr < p.T && tau_row_on(c, rr)) row[(unsigned)(c.col + rr * c.step)] = v[i];
+    }
   }
 }
 
 template <typename E>
 __device__ __forceinline__ void dtau_rows_load(const BandParams& p, const E* base, E* v, int t0w, int kb0,
                                                int lane) {
+  const TauCol c = tau_lane_col(p, t0w, kb0, lane);
 #pragma unroll
   for (int rr = 0; rr < 16; ++rr) {
-    const int t = t0w + rr;
-    const int col = t < p.T ? band_tau_col(p, t, kb0 + lane) : -1;
-    v[rr] = col >= 0 ? base[(int64_t)t * p.dtau.s1 + col] : (E)0.f;
+    // a pair without a slot reads its row's first element and is masked
+    const int t = t0w + rr < p.T ? t0w + rr : p.T - 1;
+    const bool on = t0w + rr < p.T && tau_row_on(c, rr);
+    const E x = base[(int64_t)t * p.dtau.s1 + (on ? c.col + rr * c.step : 0)];
+    v[rr] = on ? x : (E)0.f;
   }
 }
 
@@ -584,19 +608,25 @@ struct FwdTile {
   }
 };
 
-template <int NT, int NV, int D, int NORM, bool BIAS, bool TAU>
-__global__ __launch_bounds__(kThreads) void xb_fwd(BandArgs args) {
+// KS: groups of four waves per workgroup, each with every KS-th key block of the
+// band and an LDS buffer of its own; their sums meet in LDS at the end.  KS = 2 is
+// for grids that leave most wave slots empty (a prompt's prefill): a tile's chain
+// of blocks, each a round of latencies with nothing beside it, is half as long
+// (B1 H16 T777 W256, autocast types, bias and tau: 29.7 -> 24.2 us).
+template <int NT, int NV, int D, int NORM, bool BIAS, bool TAU, int KS>
+__global__ __launch_bounds__(kThreads * KS) void xb_fwd(BandArgs args) {
   touch_args(args);
   const BandParams p = band_params(args);
-  constexpr int NBUF = NT == 1 ? 2 : 1;
-  __shared__ __attribute__((aligned(16))) bf16 lds[NBUF * (NT + NV) * kDTile];
-  __shared__ __attribute__((aligned(16))) Elem<NT> tstage[TAU ? 4 * kStageRows : 1];
-  const int tid = threadIdx.x, lane = tid & 63;
+  constexpr int NBUF = NT == 1 && KS == 1 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) bf16 lds[KS * NBUF * (NT + NV) * kDTile];
+  __shared__ __attribute__((aligned(16))) Elem<NT> tstage[TAU ? 4 * KS * kStageRows : 1];
+  const int tid = threadIdx.x & (kThreads - 1), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads);
   const TileId id = tile_id(p, p.glob != 0);
   const int T = p.T;
   FwdTile<NT, NV, D, NORM, BIAS, TAU> st;
-  st.init(p, id.b, id.h, lane, wave, tstage);
+  st.init(p, id.b, id.h, lane, wave, tstage + (TAU ? grp * 4 * kStageRows : 0));
   st.at(p, id.tile * kTile);
   const Blocks bl = band_blocks(p, st.t0);
 
@@ -606,8 +636,51 @@ __global__ __launch_bounds__(kThreads) void xb_fwd(BandArgs args) {
   const Elem<NV>* vb_ = (const Elem<NV>*)p.v.p + st.b * p.v.s0 + st.h * p.v.s2;
 #pragma unroll
   for (int ch = 0; ch < D / 32; ++ch) frag_row<NT>(qb_, p.q.s1, st.tq, T, 4 * ch + st.g, st.qf[ch]);
-  stream_keys<NT, NV, D, NBUF>(lds, kb_, p.k.s1, vb_, p.v.s1, bl, T, tid,
-                           [&](const bf16* kt, int kb0) { st.visit(p, kt, kb0); });
+  if constexpr (KS == 1) {
+    stream_keys<NT, NV, D, NBUF>(lds, kb_, p.k.s1, vb_, p.v.s1, bl, T, tid,
+                                 [&](const bf16* kt, int kb0) { st.visit(p, kt, kb0); });
+  } else {
+    bf16* buf = lds + grp * (NT + NV) * kDTile;
+    if (grp < bl.n) {
+      store_raw<NT>(load_raw<NT, D>(kb_, p.k.s1, bl.first + grp * kTile, T, tid), buf, tid);
+      store_raw<NV>(load_raw<NV, D>(vb_, p.v.s1, bl.first + grp * kTile, T, tid), buf + NT * kDTile, tid);
+    }
+    __syncthreads();
+    for (int i = 0; i < bl.n; i += KS) {  // every group runs every round's barriers
+      const int kb0 = bl.first + (i + grp) * kTile;
+      const bool more = i + grp + KS < bl.n;
+      Raw<NT> kn;
+      Raw<NV> vn;
+      if (more) {
+        kn = load_raw<NT, D>(kb_, p.k.s1, kb0 + KS * kTile, T, tid);
+        vn = load_raw<NV, D>(vb_, p.v.s1, kb0 + KS * kTile, T, tid);
+      }
+      if (i + grp < bl.n) st.visit(p, buf, kb0);
+      __syncthreads();
+      if (more) {
+        store_raw<NT>(kn, buf, tid);
+        store_raw<NV>(vn, buf + NT * kDTile, tid);
+      }
+      __syncthreads();
+    }
+    static_assert(KS <= 2, "two groups meet");
+    float* red = (float*)lds + wave * (D / 4 + 1) * 64 + lane;  // D / 4 sums and the mass per lane
+    static_assert(sizeof(lds) >= 4 * (D / 4 + 1) * 64 * sizeof(float), "the sums fit the key buffers");
+    if (grp == 1) {
+#pragma unroll
+      for (int m = 0; m < D / 16; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[(4 * m + r) * 64] = st.acc[m][r];
+      red[(D / 4) * 64] = st.msum;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+#pragma unroll
+    for (int m = 0; m < D / 16; ++m)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st.acc[m][r] += red[(4 * m + r) * 64];
+    st.msum += red[(D / 4) * 64];
+  }
   st.finish(p);
 }
 
@@ -1477,8 +1550,14 @@ void launch_norm(const BandParams& p, hipStream_t st, unsigned n) {
   } while (0)
   if constexpr (PHASE == 0) {
     const bool opt = p.tau.p != nullptr;
-    if (p.chunk > 0) XB_BT(xb_fwd_run);
-    else XB_BT(xb_fwd);
+    if (p.chunk > 0) {
+      XB_BT(xb_fwd_run);
+    } else if (p.chunk < 0) {  // two key groups
+      const dim3 block(2 * kThreads);
+      XB_BT(xb_fwd, , 2);
+    } else {
+      XB_BT(xb_fwd, , 1);
+    }
   } else if constexpr (PHASE == 1) {
     const bool opt = p.dtau.p != nullptr;
     // runs of tiles (a local window W <= 64): float32 Q / K at head dim 32
