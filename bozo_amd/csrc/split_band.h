@@ -1062,8 +1062,14 @@ __device__ __forceinline__ DqTile<NT, NV, D, NORM, BIAS, DTAU> dq_tile_base(cons
   return q;
 }
 
-template <int NT, int NV, int D, int NORM, bool BIAS, bool DTAU, int MODE>
-__global__ __launch_bounds__(kThreads) void xb_dq(BandArgs args) {
+// The register budget is stated (two waves per SIMD or more): left to itself the
+// compiler spreads the accumulators over AGPRs beside the VGPRs, and the total
+// costs a wave per SIMD.  B8 H16 T1024 d64 W256, autocast types: 178 -> 162
+// registers, 108 -> 95 us; B8 H12 T1000 d64 W64 float32: 50 -> 43 us; bf16 W256
+// with dTau 109 -> 91 us.  MINW = 1 leaves it to the compiler: a float32 V over
+// wide bands (B4 H16 W256 64 against 68 us, B4 H12 global 104 against 110).
+template <int NT, int NV, int D, int NORM, bool BIAS, bool DTAU, int MODE, int MINW>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MINW, 8))) void xb_dq(BandArgs args) {
   touch_args(args);
   const BandParams p = band_params(args);
   constexpr int NBUF = (NT == 1 || MODE == 1) ? 2 : 1;
@@ -1393,8 +1399,10 @@ __device__ __forceinline__ void dkv_store(const BandParams& p, const KeyTile<NT,
 
 // Key tile k: the query tiles whose band reaches it pass through LDS in
 // turn (Q and dOut as NT terms each, plus their rows' coefficients a, c).
+// float16: the register budget as for xb_dq (B8 H16 T1024 d64 W256: 99 -> 87 us);
+// the other flows' totals stay at two waves per SIMD either way.
 template <int NT, int NV, int D, int NORM, bool BIAS, bool DTAU>
-__global__ __launch_bounds__(kThreads) void xb_dkv(BandArgs args) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NT == 2 ? 2 : 1, 8))) void xb_dkv(BandArgs args) {
   touch_args(args);
   const BandParams p = band_params(args);
   constexpr int NBUF = NT == 1 ? 2 : 1;
@@ -1460,8 +1468,11 @@ __global__ __launch_bounds__(kThreads) void xb_dkv(BandArgs args) {
 // visits query tile k + 1, then k): two runs that share a boundary query
 // tile then read it at the same time (both at their ends or both at their
 // starts), and the second read is an L2 hit.
+// With a float32 V the register budget is stated: left to the compiler the kernel
+// took 272 registers, one wave per SIMD, and one tile per workgroup was faster
+// (B8 H12 T1000 d64 W64: 54 us; the runs at two waves 45 us).
 template <int NT, int NV, int D, int NORM, bool BIAS, bool DTAU>
-__global__ __launch_bounds__(kThreads) void xb_dkv_run(BandArgs args) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NV == 3 ? 2 : 1, 8))) void xb_dkv_run(BandArgs args) {
   touch_args(args);
   const BandParams p = band_params(args);
   constexpr int TPB = 2 * NT;
@@ -1575,22 +1586,30 @@ void launch_norm(const BandParams& p, hipStream_t st, unsigned n) {
         return;
       }
     }
-    if constexpr (NORM != NORM_MASS_) {
-      XB_BT(xb_dq, , 0);
-    } else if constexpr (NV == 3) {
+    const bool narrow = !p.glob && p.win <= kTile;
+    if constexpr (NV == 3) {
       // float32 V: the register tau-mass mode would keep two blocks of six
       // terms in LDS (96 KB); the saved rows (one pass) or two passes
-      if (p.coef_pre) XB_BT(xb_dq, , 3);
-      else XB_BT(xb_dq, , 2);
+#define XB_DQ(M)                            \
+  do {                                      \
+    if (narrow) XB_BT(xb_dq, , M, 2);       \
+    else XB_BT(xb_dq, , M, 1);              \
+  } while (0)
+      if constexpr (NORM != NORM_MASS_) XB_DQ(0);
+      else if (p.coef_pre) XB_DQ(3);
+      else XB_DQ(2);
+#undef XB_DQ
+    } else if constexpr (NORM != NORM_MASS_) {
+      XB_BT(xb_dq, , 0, 2);
     } else if constexpr (NT == 3) {
       // a band within two blocks keeps P and dP in registers (faster than
       // one pass from saved rows at W = 64: 42 against 48 us at config 2)
-      if (!p.glob && p.win <= kTile) XB_BT(xb_dq, , 1);
-      else if (p.coef_pre) XB_BT(xb_dq, , 3);
-      else XB_BT(xb_dq, , 2);
+      if (narrow) XB_BT(xb_dq, , 1, 2);
+      else if (p.coef_pre) XB_BT(xb_dq, , 3, 2);
+      else XB_BT(xb_dq, , 2, 2);
     } else {  // bf16 / fp16 rows: the coefficients from the band (a 16-bit out would cancel)
-      if (!p.glob && p.win <= kTile) XB_BT(xb_dq, , 1);
-      else XB_BT(xb_dq, , 2);
+      if (narrow) XB_BT(xb_dq, , 1, 2);
+      else XB_BT(xb_dq, , 2, 2);
     }
   } else {
     const bool opt = p.dtau.p != nullptr;
