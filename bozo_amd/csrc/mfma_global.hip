@@ -92,16 +92,65 @@ __device__ __forceinline__ GlSlot gl_slot(int BH, int id) {
   return {id / BH, id % BH};
 }
 
-__device__ __forceinline__ int gl_tau_col(const BandParams& p, int q, int k) {
-  const int j = p.T - 1 - k;
-  return (q < p.T && k < p.T && j < p.Wtau) ? j : -1;
+// The lane index, opaque to the compiler: what is worked out from it stays in the
+// block that uses it (few blocks hold tau_local columns; kept across the whole loop,
+// their addresses cost the kernel a wave per SIMD).
+__device__ __forceinline__ int gl_opaque(int lane) {
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
+// tau_local / dtau_local of N pairs of a lane: pair e in row row(e) (a query, at
+// most T - 1) at column col(e), which exists in [0, width) (else 0).  One dtype
+// switch for all N, and branch-free loads (a pair without a slot reads column 0 and
+// is masked), so they are in flight together: with a switch and a wait for each
+// pair a block with columns was a chain of sixteen loads.  With these, gl_opaque
+// and the blocks with columns in loops of their own, gl_fwd and gl_dq with tau_local
+// run at three waves per SIMD like those without it: B8 H12 T1024, Wl 64: gl_fwd
+// 32.5 -> 29.1 us, gl_dq 47.9 -> 43.4, gl_dkv 58.1 -> 52.1; forward + backward
+// B4 H12 T2048: Wl 64 198 -> 177 us, Wl 512 256 -> 206 us.
+template <int N, typename E, typename Row, typename Col>
+__device__ __forceinline__ void gl_tau_get_t(const Buf& b, int64_t bh, int width, Row row, Col col, float* x) {
+  const E* base = (const E*)b.p + bh;
+  E v[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) v[e] = base[row(e) * b.s1 + ((unsigned)col(e) < (unsigned)width ? col(e) : 0)];
+#pragma unroll
+  for (int e = 0; e < N; ++e) x[e] = (unsigned)col(e) < (unsigned)width ? (float)v[e] : 0.f;
+}
+template <int N, typename Row, typename Col>
+__device__ __forceinline__ void gl_tau_get(const Buf& b, int64_t bh, int width, Row row, Col col, float* x) {
+  switch (b.dt) {
+    case TENSION_F32: gl_tau_get_t<N, float>(b, bh, width, row, col, x); break;
+    case TENSION_BF16: gl_tau_get_t<N, bf16>(b, bh, width, row, col, x); break;
+    case TENSION_F16: gl_tau_get_t<N, f16>(b, bh, width, row, col, x); break;
+    default: gl_tau_get_t<N, double>(b, bh, width, row, col, x); break;
+  }
+}
+// The eight pairs (j, r) of one query row: column col0 - 16 j - r.
+template <typename E>
+__device__ __forceinline__ void gl_tau_put8_t(const Buf& b, int64_t off, int col0, int width, const float (*x)[4]) {
+  E* row = (E*)b.p + off;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const unsigned col = col0 - 16 * (e >> 2) - (e & 3);
+    if (col < (unsigned)width) row[col] = (E)x[e >> 2][e & 3];
+  }
+}
+__device__ __forceinline__ void gl_tau_put8(const Buf& b, int64_t off, int col0, int width, const float (*x)[4]) {
+  switch (b.dt) {
+    case TENSION_F32: gl_tau_put8_t<float>(b, off, col0, width, x); break;
+    case TENSION_BF16: gl_tau_put8_t<bf16>(b, off, col0, width, x); break;
+    case TENSION_F16: gl_tau_put8_t<f16>(b, off, col0, width, x); break;
+    default: gl_tau_put8_t<double>(b, off, col0, width, x); break;
+  }
 }
 
 #ifndef TENSION_GL_FWD_WPE
 #define TENSION_GL_FWD_WPE 3
 #endif
-// with a bias or tau_local the per-pair operands need more registers: two
-// waves per SIMD instead of spilling
+// with a bias the per-pair operands need more registers: two waves per SIMD
+// instead of spilling
 #ifndef TENSION_GL_FWD_WPE_OPT
 #define TENSION_GL_FWD_WPE_OPT 2
 #endif
@@ -244,14 +293,14 @@ __device__ __forceinline__ void gl_fwd_tile(const BandParams& p, int tile, int b
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int key = blk * kTile + 32 * kh + 16 * j + 4 * g + r, query = t0 + dq;
           const float pv = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[i][j][r] * k2));
           pr[j][r] = (diag && 32 * kh + 16 * j + 4 * g + r > dq) ? 0.f : pv;
-          if (TB) {
-            const int col = gl_tau_col(p, query, key);
-            if (col >= 0) st<float>(p.tau, tau_off(p.tau, b, query, h, col), pr[j][r]);
-          }
         }
+      if constexpr (TB) {
+        const int l = gl_opaque(lane), tq = t0 + 32 * qh + 16 * i + (l & 15);
+        if (tq < T)
+          gl_tau_put8(p.tau, tau_off(p.tau, b, tq, h, 0), T - 1 - (blk * kTile + 32 * kh + 4 * (l >> 4)), p.Wtau, pr);
+      }
       const bf16x8 pb = pack_b(pr[0], pr[1]);
       if (i == 0) {
         tr_wait4(vr);
@@ -355,7 +404,7 @@ __device__ __forceinline__ void gl_fwd_tile(const BandParams& p, int tile, int b
 // tile per workgroup, one round of equal workgroups, measured slower.)
 template <bool BIAS, bool TAU>
 __global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(BIAS || TAU ? TENSION_GL_FWD_WPE_OPT : TENSION_GL_FWD_WPE, 8)))
+__attribute__((amdgpu_waves_per_eu(BIAS ? TENSION_GL_FWD_WPE_OPT : TENSION_GL_FWD_WPE, 8)))
 void gl_fwd(BandArgs args) {
   touch_args(args);
   const BandParams p = band_params(args);
@@ -376,7 +425,10 @@ void gl_fwd(BandArgs args) {
 // partial sums of an output row meet once, through LDS, at the end.
 
 #ifndef TENSION_GL_DQ_WPE
-#define TENSION_GL_DQ_WPE 2
+#define TENSION_GL_DQ_WPE 3
+#endif
+#ifndef TENSION_GL_DQ_WPE_OPT
+#define TENSION_GL_DQ_WPE_OPT 2
 #endif
 #ifndef TENSION_GL_DKV_WPE
 #define TENSION_GL_DKV_WPE 2
@@ -386,7 +438,7 @@ void gl_fwd(BandArgs args) {
 //   S^T = K Q^T, dP^T = V dO^T      (A = K / V rows from LDS)
 //   dQ^T += K^T G^T                  (A = K^T read transposed)
 template <bool BIAS, bool DTAU>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(TENSION_GL_DQ_WPE, 8)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BIAS ? TENSION_GL_DQ_WPE_OPT : TENSION_GL_DQ_WPE, 8)))
 void gl_dq(BandArgs args) {
   touch_args(args);
   const BandParams p = band_params(args);
@@ -496,19 +548,23 @@ void gl_dq(BandArgs args) {
       float gd[2][4];
       const int dq = 32 * qh + 16 * i + c;
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j) {
+        float dtl[4];
+        if constexpr (TB) {
+          const int l = gl_opaque(lane), tq = t0 + 32 * qh + 16 * i + (l & 15), row = tq < T ? tq : T - 1;
+          const int col = T - 1 - (blk * kTile + 32 * kh + 16 * j + 4 * (l >> 4));
+          gl_tau_get<4>(p.dtau, b * p.dtau.s0 + h * p.dtau.s2, p.Wtau, [&](int) { return row; },
+                        [&](int e) { return col - e; }, dtl);
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int key = blk * kTile + 32 * kh + 16 * j + 4 * g + r, query = t0 + dq;
           const float x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[i][j][r] * k2));
           float dt = dp[i][j][r] * ca[i] - cc[i];
-          if (TB) {
-            const int col = gl_tau_col(p, query, key);
-            if (col >= 0) dt += ld<float>(p.dtau, tau_off(p.dtau, b, query, h, col));
-          }
+          if (TB) dt += dtl[r];
           const float gv = dt * (x - x * x);
           gd[j][r] = (diag && 32 * kh + 16 * j + 4 * g + r > dq) ? 0.f : gv;
         }
+      }
       const bf16x8 pb = pack_b(gd[0], gd[1]);
       if (i == 0) {
         tr_wait4(kr);
@@ -519,31 +575,30 @@ void gl_dq(BandArgs args) {
       for (int m = 0; m < 4; ++m) acc[i][m] = mfma(kt[m], pb, acc[i][m]);
     }
   };
-  auto visit = [&](int blk, auto diag_tag) __attribute__((always_inline)) {  // as in the forward
-    if constexpr (DTAU) {
-      if ((blk + 1) * kTile > T - p.Wtau) {
-        block(blk, diag_tag, std::true_type{});
-        return;
-      }
-    }
-    block(blk, diag_tag, std::false_type{});
-  };
-  for (int blk = 0; blk + 1 < nblk; ++blk) {  // as in the forward
+  auto step = [&](int blk, auto tau_tag) __attribute__((always_inline)) {  // as in the forward
     wait_vm<4>();
     lds_barrier();
-    visit(blk, std::false_type{});
+    block(blk, std::false_type{}, tau_tag);
     if (BIAS || blk + 2 < nblk) {
       const int nb = blk + 2 < nblk ? blk + 2 : nblk - 1;
       lds_barrier();
       tile_async_src(ksrc, nb * kTile, Kb[blk & 1], wave);
       tile_async_src(vsrc, nb * kTile, Vb[blk & 1], wave);
     }
-  }
+  };
+  // dtau_local columns are keys T - Wtau .. T - 1: the blocks from tb on, in a
+  // loop of their own
+  const int tb = DTAU ? (T - p.Wtau) / kTile : nblk;
+  int blk0 = 0;
+  for (; blk0 + 1 < nblk && blk0 < tb; ++blk0) step(blk0, std::false_type{});
+  if constexpr (DTAU)
+    for (; blk0 + 1 < nblk; ++blk0) step(blk0, std::true_type{});
   // with a bias and nblk > 1 the last copy (of block nblk - 1 again, into
   // the other slot) may stay in flight until the merge below
   if (BIAS && nblk > 1) wait_vm<4>(); else wait_vm<0>();
   lds_barrier();
-  visit(nblk - 1, std::true_type{});
+  if (DTAU && nblk > tb) block(nblk - 1, std::true_type{}, std::true_type{});
+  else block(nblk - 1, std::true_type{}, std::false_type{});
   if constexpr (BIAS) wait_vm<0>();  // the merge reuses the ring's LDS
 
   // key halves meet (as in the forward): 16 floats per lane
@@ -751,21 +806,25 @@ void gl_dkv(BandArgs args) {
       float pa[2][4], gd[2][4];
       const int dk_ = 32 * kh + 16 * i + c;  // key - k0 (= key - q0 on the diagonal block)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j) {
+        float dtl[4];
+        if constexpr (TB) {
+          const int l = gl_opaque(lane), col = T - 1 - (k0 + 32 * kh + 16 * i + (l & 15));
+          const int q0 = (q_first + blk) * kTile + 32 * qh + 16 * j + 4 * (l >> 4);
+          gl_tau_get<4>(p.dtau, b * p.dtau.s0 + h * p.dtau.s2, p.Wtau,
+                        [&](int e) { return q0 + e < T ? q0 + e : T - 1; }, [&](int) { return col; }, dtl);
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int query = (q_first + blk) * kTile + 32 * qh + 16 * j + 4 * g + r, key = k0 + dk_;
           const float b2 = BIAS ? -kLog2e * b2n[i][j][r] : 0.f;
           const float x = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(fmaf(s[j][i][r], k2, b2)));
           const bool off = diag && 32 * qh + 16 * j + 4 * g + r < dk_;  // query before key
           float dt = dp[j][i][r] * a4[j][r] - c4[j][r];
-          if (TB) {
-            const int col = gl_tau_col(p, query, key);
-            if (col >= 0) dt += ld<float>(p.dtau, tau_off(p.dtau, b, query, h, col));
-          }
+          if (TB) dt += qrow + 16 * j + r < T ? dtl[r] : 0.f;
           pa[j][r] = off ? 0.f : x * a4[j][r];
           gd[j][r] = off ? 0.f : dt * (x - x * x);
         }
+      }
       const bf16x8 pb = pack_b(pa[0], pa[1]);
       const bf16x8 gbv = pack_b(gd[0], gd[1]);
       if (i == 0) {
@@ -802,35 +861,29 @@ void gl_dkv(BandArgs args) {
   // coefficient ring writes (lgkmcnt(0) before each).
   // dtau_local columns are keys T - Wtau .. T - 1: only key tiles that hold
   // one run the per-pair column code
-  const bool kt_tau = DTAU && k0 + kTile > T - p.Wtau;
-  auto visit = [&](int blk, auto diag_tag) __attribute__((always_inline)) {
-    if constexpr (DTAU) {
-      if (kt_tau) {
-        block(blk, diag_tag, std::true_type{});
-        return;
-      }
+  auto blocks = [&](auto tau_tag) __attribute__((always_inline)) {
+    if (nblk == 1) {
+      wait_vm<0>();
+      lds_barrier();
+      block(0, std::true_type{}, tau_tag);
+      return;
     }
-    block(blk, diag_tag, std::false_type{});
-  };
-  if (nblk == 1) {
-    wait_vm<0>();
-    lds_barrier();
-    visit(0, std::true_type{});
-  } else {
     wait_vm<4>();
     lds_barrier();
-    visit(0, std::true_type{});
+    block(0, std::true_type{}, tau_tag);
     refill(0);
     for (int blk = 1; blk + 1 < nblk; ++blk) {
       wait_vm<4>();
       lds_barrier();
-      visit(blk, std::false_type{});
+      block(blk, std::false_type{}, tau_tag);
       refill(blk);
     }
     wait_vm<0>();
     lds_barrier();
-    visit(nblk - 1, std::false_type{});
-  }
+    block(nblk - 1, std::false_type{}, tau_tag);
+  };
+  if (DTAU && k0 + kTile > T - p.Wtau) blocks(std::integral_constant<bool, DTAU>{});
+  else blocks(std::false_type{});
 
   // query halves meet: wave (kh, qh) keeps key tile i = qh and hands tile
   // 1 - qh to its partner (kh, 1 - qh): 32 floats per lane (dK, dV)
