@@ -178,7 +178,7 @@ bool split_side(int kind, const tension_buf* b) { return !b || b->dtype == split
 
 // bf16 local windows wider than one 64-row tile: without side operands (bias,
 // tau, dTau) on the wide band kernels (mfma_wide.hip); with them on the split
-// kernels.  Forward + backward at B8 H16 T1024 W256, valid count: 109 us there,
+// kernels.  Forward + backward at B8 H16 T1024 W256, valid count: 106 us there,
 // 117 us on the split kernels.
 bool wide_on_split(bool global, int64_t W, bool side) { return !global && W > 64 && side; }
 

@@ -12,7 +12,7 @@
 // W = 256, the merge) at two or three workgroups per CU, over an HBM floor of 13
 // to 20 us.  B8 H16 T1024 W256, valid count, one box (split kernels -> these):
 // forward 33.6 -> 28.5 us, dQ 46.0 -> 40.4, dK / dV 52.1 -> 52.0; forward +
-// backward 116.6 -> 109.4 us on another.
+// backward 116.6 -> 106.3 us.
 #include <type_traits>
 
 #include "mfma_common.h"
