@@ -67,23 +67,26 @@ int dtype_code(const Tensor& t) {
   }
 }
 
-// One tensor's descriptor; get() is null for an absent tensor.
+// One tensor's descriptor; get() is null for an absent tensor.  `written`: the
+// kernels write it, so a lazily cloned tensor gets memory of its own first (its
+// storage is shared until a mutable pointer is taken).
 struct Buf {
   tension_buf b{};
   bool on = false;
   Buf() = default;
-  explicit Buf(const Tensor& t) {
+  explicit Buf(const Tensor& t, bool written = false) {
     if (!t.defined()) return;
     const int code = dtype_code(t);
     if (code < 0) throw py::type_error(std::string("unsupported dtype ") + c10::toString(t.scalar_type()));
     if (t.dim() > 4) throw py::value_error("a tension_buf describes at most 4 dimensions");
     on = true;
-    b.ptr = const_cast<void*>(t.const_data_ptr());
+    b.ptr = written ? t.mutable_data_ptr() : const_cast<void*>(t.const_data_ptr());
     b.dtype = code;
     for (int64_t i = 0; i < t.dim(); ++i) b.s[i] = t.stride(i);
   }
   const tension_buf* get() const { return on ? &b : nullptr; }
 };
+Buf written(const Tensor& t) { return Buf(t, true); }
 
 // Unit innermost stride is all the kernels need.
 Tensor rows(const Tensor& t) {
@@ -143,7 +146,7 @@ std::tuple<Tensor, Tensor, Tensor> window_fwd(const Tensor& Q, const Tensor& K, 
   Tensor out = empty(Q.sizes(), Q), tau, mass;
   if (want_tau) tau = empty({B, T, H, W}, Q);
   if (want_mass) mass = empty({B, T, H}, at::kFloat, Q);
-  const Buf q(Q), k(K), v(V), o(out), t(tau), b(bias), m(mass);
+  const Buf q(Q), k(K), v(V), o = written(out), t = written(tau), b(bias), m = written(mass);
   check(tension_window_fwd(q.get(), k.get(), v.get(), o.get(), t.get(), b.get(), m.get(), B, T, H, D, W, scale,
                            (int32_t)flags, stream_of(Q)),
         "tension_window_fwd");
@@ -158,7 +161,7 @@ std::tuple<Tensor, Tensor, Tensor> window_bwd(const Tensor& Q, const Tensor& K, 
   const Tensor dOut = d_out.defined() ? rows(d_out) : at::zeros_like(Q), dTau = rows(d_tau);
   Tensor dQ = empty(Q.sizes(), Q), dK = empty(K.sizes(), K), dV = empty(V.sizes(), V);
   const Tensor ws = workspace(tension_window_bwd_workspace(B, T, H, acc_code(Q, K, V), (int32_t)flags), Q);
-  const Buf q(Q), k(K), v(V), go(dOut), gt(dTau), b(bias), gq(dQ), gk(dK), gv(dV);
+  const Buf q(Q), k(K), v(V), go(dOut), gt(dTau), b(bias), gq = written(dQ), gk = written(dK), gv = written(dV);
   if (out.defined()) {
     const Buf o(out), m(mass);
     check(tension_window_bwd_saved(q.get(), k.get(), v.get(), go.get(), gt.get(), b.get(), o.get(), m.get(), gq.get(),
@@ -208,7 +211,7 @@ std::tuple<Tensor, Tensor, Tensor> global_fwd(const Tensor& Q, const Tensor& K, 
   Tensor out = at::empty_like(Q), tl;
   if (Wl > 0) tl = empty({B, T, H, Wl}, Q);
   Tensor mass = empty({B, T, H}, at::kFloat, Q);
-  const Buf q(Q), k(K), v(V), o(out), t(tl), b(bias), m(mass);
+  const Buf q(Q), k(K), v(V), o = written(out), t = written(tl), b(bias), m = written(mass);
   check(tension_global_fwd(q.get(), k.get(), v.get(), o.get(), t.get(), b.get(), m.get(), B, T, H, D, Wl, scale, 0,
                            stream_of(Q)),
         "tension_global_fwd");
@@ -224,7 +227,8 @@ std::tuple<Tensor, Tensor, Tensor> global_bwd(const Tensor& Q, const Tensor& K, 
   const Tensor dTl = Wl > 0 ? rows(d_tl) : Tensor();
   Tensor dQ = empty(Q.sizes(), Q), dK = empty(K.sizes(), K), dV = empty(V.sizes(), V);
   const Tensor ws = workspace(tension_global_bwd_workspace(B, T, H, acc_code(Q, K, V), 0), Q);
-  const Buf q(Q), k(K), v(V), go(dOut), gt(dTl), b(bias), o(out), m(mass), gq(dQ), gk(dK), gv(dV);
+  const Buf q(Q), k(K), v(V), go(dOut), gt(dTl), b(bias), o(out), m(mass), gq = written(dQ), gk = written(dK),
+      gv = written(dV);
   check(tension_global_bwd(q.get(), k.get(), v.get(), go.get(), gt.get(), b.get(), o.get(), m.get(), gq.get(),
                            gk.get(), gv.get(), ptr(ws), B, T, H, D, Wl, scale, 0, stream_of(Q)),
         "tension_global_bwd");
@@ -259,7 +263,7 @@ Tensor rope_call(const Tensor& x, const Tensor& cos, const Tensor& sin, int64_t 
                  int64_t inverse) {
   const c10::DeviceGuard guard(x.device());
   Tensor y = empty(x.sizes(), out_dtype, x);
-  const Buf bx(x), by(y);
+  const Buf bx(x), by = written(y);
   check(tension_rope(bx.get(), by.get(), cos.data_ptr<float>(), sin.data_ptr<float>(), cos.size(0), x.size(0),
                      x.size(1), x.size(2), x.size(3), pos_offset, (int32_t)inverse, stream_of(x)),
         "tension_rope");
@@ -310,10 +314,13 @@ OptTensor decode_step(const Tensor& q, const Tensor& kn, const Tensor& vn, const
   const c10::DeviceGuard guard(q.device());
   Tensor out = at::empty_like(q);
   const Tensor qr = rows(q), knr = rows(kn), vnr = rows(vn);
-  const Buf bq(qr), bkn(knr), bvn(vnr), bkc(kc), bvc(vc), bo(out), bt(tau);
+  // the caller's own tensors, appended to and written in place; taken ahead of
+  // the operands that are read, which may be views of the same storage
+  const Buf bkc = written(kc), bvc = written(vc), bt = written(tau), bo = written(out);
+  int32_t* const pout = pos_out.defined() ? pos_out.mutable_data_ptr<int32_t>() : nullptr;
+  const Buf bq(qr), bkn(knr), bvn(vnr);
   check(tension_decode_step(bq.get(), bkn.get(), bvn.get(), bkc.get(), bvc.get(), bo.get(), bt.get(),
-                            pos_in.data_ptr<int32_t>(), pos_out.defined() ? pos_out.data_ptr<int32_t>() : nullptr, N,
-                            H, D, W, scale, (int32_t)flags, stream_of(q)),
+                            pos_in.const_data_ptr<int32_t>(), pout, N, H, D, W, scale, (int32_t)flags, stream_of(q)),
         "tension_decode_step");
   return out;
 }
