@@ -8,6 +8,12 @@
 // LDS, at the end.  Only the blocks that cross a band edge are masked, and a
 // wave skips the 32 x 32 quarters that lie outside.
 //
+// A masked pair enters the second products as weight 0 times its row, so an
+// infinity or NaN in that row would reach the result.  Products are left out 16
+// result rows x 32 summed rows at a time where no pair of the group lies on the
+// band, the same groups as in the split kernels: a non-finite row reaches the
+// result rows it has a pair with and those that share such a group with it.
+//
 // Bound by each workgroup's own latencies (first loads, five dependent blocks at
 // W = 256, the merge) at two or three workgroups per CU, over an HBM floor of 13
 // to 20 us.  B8 H16 T1024 W256, valid count, one box (split kernels -> these):
@@ -20,9 +26,13 @@
 namespace tension {
 namespace {
 
-// Band of a wave's 32 queries [qa, qa + 31] against 32 keys [ka, ka + 31]
-// (query t sees keys t - W .. t - 1, t < T): outside, crossing an edge, inside.
-__device__ __forceinline__ bool quarter_out(int qa, int ka, int W) { return ka > qa + 30 || ka + 31 < qa - W; }
+// No pair of NQ queries from qa and NK keys from ka on the band (query t sees
+// keys t - W .. t - 1).  In a 32 x 32 quarter that has pairs, 16 rows without any
+// can only lie past the band's far edge: the later queries, or the earlier keys.
+template <int NQ, int NK>
+__device__ __forceinline__ bool pairs_out(int qa, int ka, int W) {
+  return ka > qa + NQ - 2 || ka + NK - 1 < qa - W;
+}
 
 __device__ __forceinline__ bool pair_on(int q, int k, int W) { return k < q && k >= q - W; }
 
@@ -147,6 +157,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 8))
     bf16x8 vt[4];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
+      if (MASK && i == 1 && pairs_out<16, 32>(qa + 16, ka, W)) break;
       float pr[2][4];
       const int q = qa + 16 * i + c;
 #pragma unroll
@@ -169,7 +180,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 8))
   };
   ring<0>(ks, vs, key_blocks(p, id.tile), lds, wave, [](int, int) {}, [&](int blk, int slot) __attribute__((always_inline)) {
     const int ka = blk * kTile + 32 * kh;
-    if (quarter_out(qa, ka, W)) return;
+    if (pairs_out<32, 32>(qa, ka, W)) return;
     if (ka + 31 < qa && ka >= qa + 31 - W) block(lds[slot], lds[kRing + slot], ka, std::false_type{});
     else block(lds[slot], lds[kRing + slot], ka, std::true_type{});
   });
@@ -229,7 +240,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))
   auto each = [&](auto body) __attribute__((always_inline)) {
     ring<0>(ks, vs, kr, lds, wave, [](int, int) {}, [&](int blk, int slot) __attribute__((always_inline)) {
       const int ka = blk * kTile + 32 * kh;
-      if (quarter_out(qa, ka, W)) return;
+      if (pairs_out<32, 32>(qa, ka, W)) return;
       if (ka + 31 < qa && ka >= qa + 31 - W) body(lds[slot], lds[kRing + slot], ka, std::false_type{});
       else body(lds[slot], lds[kRing + slot], ka, std::true_type{});
     });
@@ -293,6 +304,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))
     bf16x8 kt[4];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
+      if (MASK && i == 1 && pairs_out<16, 32>(qa + 16, ka, W)) break;
       float gd[2][4];
 #pragma unroll
       for (int j = 0; j < 2; ++j)
@@ -417,6 +429,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))
           gt[m] = tr_join(gt_[m]);
         }
       }
+      // (left out from the pairs' arithmetic on, in either order of i, the kernel
+      // spills 12 to 27 registers; so only the products are)
+      if (MASK && i == 0 && pairs_out<32, 16>(qa, ka, W)) continue;
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         dv[i][m] = mfma(gt[m], pb, dv[i][m]);
@@ -426,7 +441,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 8))
   };
   ring<NORM == NORM_MASS_ ? 1 : 0>(qs, gs, qr, tiles, wave, coef_copy, [&](int blk, int slot) __attribute__((always_inline)) {
     const int qa = blk * kTile + 32 * qh;
-    if (quarter_out(qa, ka, W)) return;
+    if (pairs_out<32, 32>(qa, ka, W)) return;
     if (ka + 31 < qa && ka >= qa + 31 - W && qa + 31 < T) block(tiles[slot], tiles[kRing + slot], coef[slot], qa, std::false_type{});
     else block(tiles[slot], tiles[kRing + slot], coef[slot], qa, std::true_type{});
   });
