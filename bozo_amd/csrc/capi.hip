@@ -176,11 +176,45 @@ bool split_dv_rows(int kind, const tension_buf* b) {
 // them as typed rows).
 bool split_side(int kind, const tension_buf* b) { return !b || b->dtype == split_qk_dtype(kind); }
 
-// bf16 local windows wider than one 64-row tile: without side operands (bias,
-// tau, dTau) on the wide band kernels (mfma_wide.hip); with them on the split
-// kernels.  Forward + backward at B8 H16 T1024 W256, valid count: 106 us there,
-// 117 us on the split kernels.
-bool wide_on_split(bool global, int64_t W, bool side) { return !global && W > 64 && side; }
+// bf16 local windows wider than one 64-row tile: with side operands (bias, tau,
+// dTau) on the split kernels; without them, phase by phase (0 forward, 1 dQ, 2
+// dK / dV; the two kernel sets keep the same coefficients in the workspace), on
+// whichever of those and the wide band kernels (mfma_wide.hip) is faster.
+//
+// The wide kernels read half the LDS per product and copy by DMA; the split
+// kernels cut the band's edges into pieces half as large, and their backward
+// holds three workgroups per CU where wl_dq and wl_dkv hold two.  So the wide
+// kernels win from where the edges are a small part of the band, the earlier the
+// better their rounds come out: four workgroups per CU are two rounds on either,
+// three are one round against two.  Least window at which they are no slower, by
+// workgroups per CU (measured at H16 T1024, sustained, tau mass and valid count;
+// split -> wide, us, tau mass):
+//   2 per CU   fwd W96 8.5 -> 8.4    dQ W96 13.9 -> 13.4     dK/dV W128 12.3 -> 11.8
+//   3          fwd W96 10.4 -> 10.5  dQ W320 30.1 -> 29.6    dK/dV W384 26.6 -> 27.2
+//   4          fwd W128 13.0 -> 13.2 dQ W256 31.6 -> 30.6    dK/dV W128 22.6 -> 21.3
+//   6          fwd W128 18.2 -> 17.1 dQ W256 47.2 -> 44.0    dK/dV W256 37.4 -> 37.1
+//   8          fwd W128 21.2 -> 21.2 dQ W320 63.6 -> 63.3    dK/dV W128 40.1 -> 37.5
+//              (W80: 19.7 -> 21.6    W128 37.7 -> 43.6       W80 36.5 -> 39.2)
+//   16         fwd W128 41.6 -> 41.6 dQ W512 157 -> 152      dK/dV W320 105 -> 105
+//   24         fwd W128 59.4 -> 60.5 dQ W512 226 -> 222      dK/dV W384 165 -> 165
+//              (W80: 56.5 -> 60.9    W256 150 -> 167         W128 102 -> 113)
+int64_t wide_from(int phase, int64_t workgroups) {
+  const int64_t cus = device_cus(), per_cu = (workgroups + cus - 1) / cus;
+  static const struct {
+    int64_t upto, from[3];
+  } rule[] = {{2, {96, 96, 128}},  {3, {96, 320, 384}},   {4, {128, 256, 128}},       {6, {128, 256, 256}},
+              {8, {128, 320, 128}}, {16, {128, 512, 320}}, {INT64_MAX, {128, 512, 384}}};
+  int i = 0;
+  while (per_cu > rule[i].upto) ++i;
+  return rule[i].from[phase];
+}
+
+bool wide_on_split(int phase, bool global, Shape sh, int64_t W, bool side) {
+  if (global || W <= 64) return false;
+  if (side) return true;
+  const int64_t n = sh.B * sh.H * ((sh.T + 63) / 64);
+  return n > device_cus() && (W < sh.T ? W : sh.T) < wide_from(phase, n);
+}
 
 enum {
   KERNEL_EXACT = 0,
@@ -257,7 +291,7 @@ int band_fwd(const tension_buf* q, const tension_buf* k, const tension_buf* v, c
   bool mf = !(flags & TENSION_FORCE_EXACT) && sh.D == 64 && aligned_bf16_rows(q) && aligned_bf16_rows(k) &&
                   aligned_bf16_rows(v) && aligned_bf16_rows(out) && (!bias || bias->dtype == TENSION_F32);
   // (the wide kernels write the tau mass only where it normalises)
-  if (wide_on_split(global, Wparam, bias || tau || (mass && !(flags & TENSION_NORM_MASS)))) mf = false;
+  if (mf && wide_on_split(0, global, sh, Wparam, bias || tau || (mass && !(flags & TENSION_NORM_MASS)))) mf = false;
   const int sk = mf ? SPLIT_NONE : split_kind(q, k, v, bias, sh.D, flags);
   const bool sp = sk != SPLIT_NONE && split_rows(sk, out) && split_side(sk, tau);
   return run_band(0, sp ? split_kernel(sk) : mf ? KERNEL_MFMA : KERNEL_EXACT, any_f64(q, k, v), p, stream, what);
@@ -335,7 +369,7 @@ int band_bwd_dq(const tension_buf* q, const tension_buf* k, const tension_buf* v
   BandParams p = bwd_params(q, k, v, dout, dtau, bias, ws, sh, Wparam, scale, flags, global);
   p.dq = make_buf(dq);
   bool mf = mfma_ok_bwd(q, k, v, dout, bias, dq, nullptr, sh.D, flags);
-  if (wide_on_split(global, Wparam, bias || dtau)) mf = false;
+  if (mf && wide_on_split(1, global, sh, Wparam, bias || dtau)) mf = false;
   const int sk = mf ? SPLIT_NONE : split_kind(q, k, v, bias, sh.D, flags);
   const bool sp = sk != SPLIT_NONE && split_rows(sk, dout) && split_rows(sk, dq) && split_side(sk, dtau);
   // the forward's saved output rows and tau mass (the tau-mass coefficients
@@ -372,7 +406,7 @@ int band_bwd_dkv(const tension_buf* q, const tension_buf* k, const tension_buf* 
   p.dk = make_buf(dk);
   p.dv = make_buf(dv);
   bool mf = mfma_ok_bwd(q, k, v, dout, bias, dk, dv, sh.D, flags);
-  if (wide_on_split(global, Wparam, bias || dtau)) mf = false;
+  if (mf && wide_on_split(2, global, sh, Wparam, bias || dtau)) mf = false;
   const int sk = mf ? SPLIT_NONE : split_kind(q, k, v, bias, sh.D, flags);
   const bool sp = sk != SPLIT_NONE && split_rows(sk, dout) && split_rows(sk, dk) && split_dv_rows(sk, dv) &&
                   split_side(sk, dtau);

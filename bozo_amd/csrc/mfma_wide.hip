@@ -16,9 +16,10 @@
 //
 // Bound by each workgroup's own latencies (first loads, five dependent blocks at
 // W = 256, the merge) at two or three workgroups per CU, over an HBM floor of 13
-// to 20 us.  B8 H16 T1024 W256, valid count, one box (split kernels -> these):
-// forward 33.6 -> 28.5 us, dQ 46.0 -> 40.4, dK / dV 52.1 -> 52.0; forward +
-// backward 116.6 -> 106.3 us.
+// to 20 us.  B8 H16 T1024 W256, valid count, sustained (split kernels -> these):
+// forward 28.1 -> 25.1 us, dQ 33.8 -> 35.5, dK / dV 49.5 -> 45.7.  Which calls
+// take them, phase by phase: wide_from in capi.hip; forward + backward of that
+// call, with dQ on the split kernels, 106.5 -> 104.8 us.
 #include <type_traits>
 
 #include "mfma_common.h"
