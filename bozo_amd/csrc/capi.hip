@@ -203,7 +203,7 @@ int64_t wide_from(int phase, int64_t workgroups) {
   static const struct {
     int64_t upto, from[3];
   } rule[] = {{2, {96, 96, 128}},  {3, {96, 320, 384}},   {4, {128, 256, 128}},       {6, {128, 256, 256}},
-              {8, {128, 320, 128}}, {16, {128, 512, 320}}, {INT64_MAX, {128, 512, 384}}};
+              {10, {128, 320, 128}}, {16, {128, 512, 320}}, {INT64_MAX, {128, 512, 384}}};
   int i = 0;
   while (per_cu > rule[i].upto) ++i;
   return rule[i].from[phase];
