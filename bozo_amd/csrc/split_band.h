@@ -1470,9 +1470,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NT == 
 // starts), and the second read is an L2 hit.
 // With a float32 V the register budget is stated: left to the compiler the kernel
 // took 272 registers, one wave per SIMD, and one tile per workgroup was faster
-// (B8 H12 T1000 d64 W64: 54 us; the runs at two waves 45 us).
+// (B8 H12 T1000 d64 W64: 54 us; the runs at two waves 45 us).  So is that of the
+// float16 kernels at head dim 32 with a dTau or a bias, which the compiler left
+// 2 to 4 registers above three waves: one run per (b, h) from 513 (b, h) on, more
+// than two workgroups per CU (B40 H16 T256 W33, valid count, dTau 41.5 -> 32.9 us;
+// B32 26.3 -> 26.6).
+constexpr int dkv_run_waves(int NT, int NV, int D, int norm, bool bias, bool dtau) {
+  if (NV == 3) return 2;
+  return NT == 2 && D == 32 && bias != dtau && !(bias && norm == NORM_MASS_) ? 3 : 1;
+}
+
 template <int NT, int NV, int D, int NORM, bool BIAS, bool DTAU>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NV == 3 ? 2 : 1, 8))) void xb_dkv_run(BandArgs args) {
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(dkv_run_waves(NT, NV, D, NORM, BIAS, DTAU), 8))) void xb_dkv_run(BandArgs args) {
   touch_args(args);
   const BandParams p = band_params(args);
   constexpr int TPB = 2 * NT;
