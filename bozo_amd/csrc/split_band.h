@@ -613,8 +613,17 @@ struct FwdTile {
 // for grids that leave most wave slots empty (a prompt's prefill): a tile's chain
 // of blocks, each a round of latencies with nothing beside it, is half as long
 // (B1 H16 T777 W256, autocast types, bias and tau: 29.7 -> 24.2 us).
+// With tau at head dim 64 the register budget is stated for 16-bit rows (four
+// waves per SIMD, what its LDS admits), where the compiler left them at three:
+// float16 B8 H12 T1024 global with tau_local 98 -> 91 us, B4 H16 T1024 W256 with
+// tau 44 -> 37, with a bias 61 -> 46; bf16 with a bias 52 -> 40.
+constexpr int fwd_waves(int NT, int D, bool bias, bool tau, int ks) {
+  return ks == 1 && D == 64 && tau && (NT == 2 || (NT == 1 && bias)) ? 4 : 1;
+}
+
 template <int NT, int NV, int D, int NORM, bool BIAS, bool TAU, int KS>
-__global__ __launch_bounds__(kThreads * KS) void xb_fwd(BandArgs args) {
+__global__ __launch_bounds__(kThreads * KS) __attribute__((amdgpu_waves_per_eu(fwd_waves(NT, D, BIAS, TAU, KS), 8)))
+void xb_fwd(BandArgs args) {
   touch_args(args);
   const BandParams p = band_params(args);
   constexpr int NBUF = NT == 1 && KS == 1 ? 2 : 1;
