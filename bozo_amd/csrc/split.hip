@@ -31,7 +31,7 @@ int launch_split(int phase, int flow, const BandParams& p_in, hipStream_t st, hi
   // p.chunk > 0: runs of consecutive tiles per workgroup (p.chunk runs per
   // (b, h)) for a local window W <= 64: the forward, sized for about three
   // resident workgroups per CU, and the backward kernels for about two: dK /
-  // dV, and dQ for float32 Q / K with a bf16 V at head dim 32 without dTau
+  // dV (float32 throughout at head dim 64: see below), and dQ for float32 Q / K with a bf16 V at head dim 32 without dTau
   // (where its run kernel measured faster); 0: one tile per workgroup; -1: see
   // below
   p.chunk = 0;
@@ -39,9 +39,23 @@ int launch_split(int phase, int flow, const BandParams& p_in, hipStream_t st, hi
   if ((phase != 1 || dq_runs) && !p.glob && p.win >= 1 && p.win <= 64) {
     const int64_t bh = (int64_t)p.B * p.H;
     const int64_t per_cu = phase == 0 ? 3 : 2;
-    int64_t runs = (per_cu * (int64_t)device_cus() + bh / 2) / bh;
+    const int64_t slots = per_cu * (int64_t)device_cus();
+    int64_t runs = (slots + bh / 2) / bh;
+    bool take = true;
+    if (phase == 2 && flow == SPLIT_FLOW_F32V && p.D == 64) {
+      // the float32 kernel holds exactly two workgroups per CU, so a few runs over
+      // would be a round of their own, and the runs are worth it only where they
+      // fill their rounds: to 65%, with a bias or a dTau (where they gain less over
+      // one tile per workgroup) to 90%.  One tile -> runs, valid count, W 64, us:
+      // 96 (b, h) of T1000 51 -> 45, with dTau 59 -> 58; 128 64 -> 54, 75 -> 69; 192
+      // (three runs each, 2.25 per CU) 88 -> 99, 104 -> 135; 514 220 -> 269, 251 ->
+      // 374; 704 of T256 83 -> 77, 99 -> 102; 1024 117 -> 100, 140 -> 124.
+      runs = slots / bh;
+      const int64_t wg = bh * (runs < 1 ? 1 : runs), rounds = (wg + slots - 1) / slots;
+      take = 20 * wg >= (p.dtau.p || p.bias.p ? 18 : 13) * rounds * slots;
+    }
     if (runs < 1) runs = 1;
-    if (runs < p.ntiles) {
+    if (take && runs < p.ntiles) {
       p.chunk = (int)runs;
       nwg = bh * runs;
     }
