@@ -485,16 +485,17 @@ __global__ __launch_bounds__(64 * NW) void decode_rows(DecodeParams p) {
   for (int base = 0; base < rows; base += RPW * NW * U) {
     Row8<QT> k[U];
     Row8<VT> v[U];
-    // past the cache: its last row, unused
+    // past the rows: the last of them again, unused (rows that no token has filled
+    // are not read)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int s = base + first + u * RPW * NW;
-      k[u] = row8_load<LPR>(kb + (int64_t)(s < W ? s : W - 1) * p.kc.s2, ch);
+      k[u] = row8_load<LPR>(kb + (int64_t)(s < rows ? s : rows - 1) * p.kc.s2, ch);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int s = base + first + u * RPW * NW;
-      v[u] = row8_load<LPR>(vb + (int64_t)(s < W ? s : W - 1) * p.vc.s2, ch);
+      v[u] = row8_load<LPR>(vb + (int64_t)(s < rows ? s : rows - 1) * p.vc.s2, ch);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
