@@ -446,8 +446,8 @@ __device__ __forceinline__ void row8_f32(const Row8<T>& r, float* x) {
   }
 }
 
-// Waves per workgroup: 4, or 16 for a long cache on a grid that would leave most
-// wave slots empty (kRowsU rows of K and V per lane in flight either way).
+// Waves per workgroup: 4, or 16 for a long cache on a small grid (kRowsU rows
+// of K and V per lane in flight either way).
 constexpr int kRowsU = 4;
 
 template <typename QT, typename VT, int LPR, int NW>
@@ -659,9 +659,17 @@ int launch_decode(int flow, int rows, bool f64, const DecodeParams& p_in, hipStr
 #undef DECODE_FAST
   } else {
     const dim3 grid((unsigned)(p_in.N * p_in.H));
-    // 16 waves where fewer than two workgroups per CU each have more than one
-    // 4-wave trip (64 / LPR x 4 x kRowsU rows) to make
-    const bool deep = (int64_t)p_in.N * p_in.H < 2 * device_cus() && (int64_t)p_in.W * p_in.D > 8 * 64 * 4 * kRowsU;
+    // 16 waves for a cache of two 4-wave trips or more (64 / LPR x 4 x kRowsU rows
+    // each) on a grid of at most one workgroup per CU.  A CU holds one 16-wave
+    // workgroup, so on up to two per CU the second round is worth it only for 16-bit
+    // rows and 16 trips.  4 -> 16 waves, us, all rows live: float32 D64, 192 workgroups W256 9.2 -> 9.0, W512
+    // 14.3 -> 12.1, W1024 23.8 -> 19.7, W64 5.9 -> 7.3; 288 workgroups W512 19.1 ->
+    // 21.5, W1024 32.1 -> 35.5, with 100 tokens 7.5 -> 13.1; bf16 D32, 192 workgroups
+    // W512 8.3 -> 8.0, W1024 12.0 -> 9.1; bf16 D128, 384 workgroups W512 23.9 -> 23.4,
+    // W1024 41.0 -> 38.1, W2048 77.1 -> 72.7.
+    const int64_t wgs = (int64_t)p_in.N * p_in.H, trips = (int64_t)p_in.W * p_in.D / (8 * 64 * 4 * kRowsU);
+    const bool bits16 = rows == DECODE_BF16 || rows == DECODE_F16;
+    const bool deep = wgs <= device_cus() ? trips >= 2 : bits16 && wgs < 2 * device_cus() && trips >= 16;
 #define DECODE_ROWS_D(QT, VT, LPR)                                                              \
   do {                                                                                          \
     if (deep) hipLaunchKernelGGL((decode_rows<QT, VT, LPR, 16>), grid, dim3(1024), 0, st, p_in); \
