@@ -1,8 +1,8 @@
-// bf16 MFMA band backward, dK/dV half (local window and global block), head
-// dim 64.  Key-centric: one workgroup owns a 64-key tile and the four waves
-// split its keys (16 each), so every dK/dV row is produced by exactly one
-// wave -- no atomics, deterministic.  For every 64-query block that sees
-// the tile:
+// bf16 MFMA band backward, dK/dV half (local windows W <= 64; the global block
+// takes gl_dkv), head dim 64.  Key-centric: one workgroup owns a 64-key tile
+// and the four waves split its keys (16 each), so every dK/dV row is produced
+// by exactly one wave -- no atomics, deterministic.  For every 64-query block
+// that sees the tile:
 //   S  = Q K^T,  dP = dO V^T       (A = Q / dO rows from LDS, B = this
 //                                    wave's K / V fragments)
 //   P  = sigma(S/scale + bias),  G = (a_t dP - c_t + dTau) P (1 - P)

@@ -1,6 +1,7 @@
-// bf16 MFMA band backward, dQ half (local window and global block), head
-// dim 64.  Query-centric like the forward: the four waves split the 64
-// queries of the tile.  Per 64-key block:
+// bf16 MFMA band backward, dQ half (local windows W <= 64, and the global
+// block without the forward's saved rows), head dim 64.  Query-centric like
+// the forward: the four waves split the 64 queries of the tile.  Per 64-key
+// block:
 //   S^T  = K Q^T,  dP^T = V dO^T          (A = K / V rows from LDS)
 //   G    = (a_t dP - c_t + dTau) * P (1 - P) on the band          (fp32)
 //   dQ^T += K^T G^T                        (A = K^T from a transposed tile)

@@ -20,8 +20,9 @@
 //     The slots are tiles of one LDS array selected at compile time; the
 //     ring is synchronised with fence-free barriers after explicit copy
 //     waits, so reads of one slot do not wait on the DMA into another.
-//   mfma_fwd (any band, including the global block): one tile per workgroup,
-//     key blocks streamed through a two-deep ring.
+//   mfma_fwd (the global block, for K / V rows too far apart for gl_fwd's
+//     32-bit tile offsets): one tile per workgroup, key blocks streamed
+//     through a two-deep ring.
 #include "mfma_common.h"
 
 namespace tension {
@@ -496,9 +497,9 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd_ring(BandArgs args) {
   }
 }
 
-// ------------------------------------------------------------------ streaming kernel
+// ------------------------------------------------------------------ streaming kernel (global)
 
-template <int NORM, bool BIAS, bool TAU>
+template <bool BIAS, bool TAU>
 __global__ __launch_bounds__(kThreads) void mfma_fwd(BandArgs args) {
   touch_args(args);
   const BandParams p = band_params(args);
@@ -506,32 +507,25 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd(BandArgs args) {
   __shared__ __attribute__((aligned(16))) bf16 Vb[2][kDTile];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
-  const TileId id = tile_id(p, p.glob != 0);
+  const TileId id = tile_id(p, true);
   const int b = id.b, h = id.h, T = p.T;
   const int t0 = id.tile * kTile;
   const int tq = t0 + wave * 16 + c;
-  const int lo = tq - p.win > 0 ? tq - p.win : 0;
-  const int hi = tq < T ? tq - 1 + p.diag : -1;
+  const int lo = 0, hi = tq < T ? tq : -1;
   const WaveBand wb = wave_band(p, t0 + wave * 16);
 
   const bf16* qb_ = (const bf16*)p.q.p + b * p.q.s0 + h * p.q.s2;
   const bf16* kb_ = (const bf16*)p.k.p + b * p.k.s0 + h * p.k.s2;
   const bf16* vb_ = (const bf16*)p.v.p + b * p.v.s0 + h * p.v.s2;
 
-  int s_lo = t0 - p.win;
-  if (s_lo < 0) s_lo = 0;
-  int s_hi = t0 + kTile - 2 + p.diag;
-  if (s_hi > T - 1) s_hi = T - 1;
-  const int kb_first = s_lo & ~(kTile - 1);
-  const int nblk = s_hi < kb_first ? 0 : (s_hi - kb_first) / kTile + 1;
-
+  const int nblk = id.tile + 1;
   bf16x8 qf[2];
   load_qfrag(qb_, p.q.s1, tq, T, g, qf);
-  tile_async(kb_, p.k.s1, kb_first, T, Kb[0], wave, lane);
-  tile_async(vb_, p.v.s1, kb_first, T, Vb[0], wave, lane);
+  tile_async(kb_, p.k.s1, 0, T, Kb[0], wave, lane);
+  tile_async(vb_, p.v.s1, 0, T, Vb[0], wave, lane);
   if (nblk > 1) {
-    tile_async(kb_, p.k.s1, kb_first + kTile, T, Kb[1], wave, lane);
-    tile_async(vb_, p.v.s1, kb_first + kTile, T, Vb[1], wave, lane);
+    tile_async(kb_, p.k.s1, kTile, T, Kb[1], wave, lane);
+    tile_async(vb_, p.v.s1, kTile, T, Vb[1], wave, lane);
   }
   if (tq >= T) { qf[0] = bf16x8{}; qf[1] = bf16x8{}; }
   const float k2 = -kLog2e * (float)(1.0 / p.scale);
@@ -539,7 +533,7 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd(BandArgs args) {
   f32x4 macc = {};
   float msum = 0.f;
   for (int blk = 0; blk < nblk; ++blk) {
-    const int kb0 = kb_first + blk * kTile;
+    const int kb0 = blk * kTile;
     if (blk + 1 < nblk) wait_vm<4>(); else wait_vm<0>();
     __syncthreads();
     float braw[BIAS ? 4 : 1][4];
@@ -552,66 +546,71 @@ __global__ __launch_bounds__(kThreads) void mfma_fwd(BandArgs args) {
       tile_async(vb_, p.v.s1, kb0 + 2 * kTile, T, Vb[blk & 1], wave, lane);
     }
   }
-  fwd_epilogue<NORM, TAU>(p, b, h, tq, g, acc, macc[0], true);
+  fwd_epilogue<NORM_MASS_, TAU>(p, b, h, tq, g, acc, macc[0], true);
 }
 
 // ------------------------------------------------------------------ launch
 
 template <int NORM, bool BIAS, bool TAU>
-static void go(const BandParams& p, hipStream_t st, unsigned nwg, bool ring) {
-  if (ring) {
-    const unsigned n = (unsigned)((int64_t)p.B * p.H * ((p.ntiles + p.chunk - 1) / p.chunk));
+static void go(const BandParams& p, hipStream_t st) {
+  const unsigned n = (unsigned)((int64_t)p.B * p.H * ((p.ntiles + p.chunk - 1) / p.chunk));
+  BandArgs a;
+  if (!band_args(p, &a)) return;  // the host takes the ring kernel only with 32-bit strides
 #ifndef TENSION_NO_FAST_FWD
-    // the staged output stores need a free ring slot: at most two tiles per
-    // workgroup
-    // with tau: bf16 rows of 64 slots, 16-byte aligned (staged stores)
-    const Buf& tb = p.tau;
-    const bool tau_rows = !TAU || (tb.dt == TENSION_BF16 && ((tb.s0 | tb.s1 | tb.s2) & 7) == 0 &&
-                                   ((uintptr_t)tb.p & 15) == 0);
-    BandArgs a;
-    if (!band_args(p, &a)) return;  // the host takes the ring kernel only with 32-bit strides
-    if (tau_rows && p.win == kTile && p.T % kTile == 0) {
-      if (a.chunk > 2) a.chunk = 2;
-      const unsigned nq = (unsigned)((int64_t)a.B * a.H * ((a.ntiles + a.chunk - 1) / a.chunk));
-      hipLaunchKernelGGL((mfma_fwd_ring<NORM, BIAS, TAU, true>), dim3(nq), dim3(kThreads), 0, st, a);
-      return;
-    }
-#else
-    BandArgs a;
-    if (!band_args(p, &a)) return;
-#endif
-    hipLaunchKernelGGL((mfma_fwd_ring<NORM, BIAS, TAU, false>), dim3(n), dim3(kThreads), 0, st, a);
-  } else {
-    hipLaunchKernelGGL((mfma_fwd<NORM, BIAS, TAU>), dim3(nwg), dim3(kThreads), 0, st, to_args(p));
+  // the staged output stores need a free ring slot: at most two tiles per
+  // workgroup
+  // with tau: bf16 rows of 64 slots, 16-byte aligned (staged stores)
+  const Buf& tb = p.tau;
+  const bool tau_rows = !TAU || (tb.dt == TENSION_BF16 && ((tb.s0 | tb.s1 | tb.s2) & 7) == 0 &&
+                                 ((uintptr_t)tb.p & 15) == 0);
+  if (tau_rows && p.win == kTile && p.T % kTile == 0) {
+    if (a.chunk > 2) a.chunk = 2;
+    const unsigned nq = (unsigned)((int64_t)a.B * a.H * ((a.ntiles + a.chunk - 1) / a.chunk));
+    hipLaunchKernelGGL((mfma_fwd_ring<NORM, BIAS, TAU, true>), dim3(nq), dim3(kThreads), 0, st, a);
+    return;
   }
+#endif
+  hipLaunchKernelGGL((mfma_fwd_ring<NORM, BIAS, TAU, false>), dim3(n), dim3(kThreads), 0, st, a);
 }
 
 template <int NORM>
-static void go_n(const BandParams& p, hipStream_t st, unsigned nwg, bool bias, bool tau, bool ring) {
+static void go_n(const BandParams& p, hipStream_t st, bool bias, bool tau) {
   if (bias) {
-    if (tau) go<NORM, true, true>(p, st, nwg, ring); else go<NORM, true, false>(p, st, nwg, ring);
+    if (tau) go<NORM, true, true>(p, st); else go<NORM, true, false>(p, st);
   } else {
-    if (tau) go<NORM, false, true>(p, st, nwg, ring); else go<NORM, false, false>(p, st, nwg, ring);
+    if (tau) go<NORM, false, true>(p, st); else go<NORM, false, false>(p, st);
   }
 }
 
 void launch_gl_fwd(const BandParams& p, hipStream_t st);
 
+// A local window of at most a tile (wider ones take other kernels), or the
+// global block (tau-mass normalised always).
 void launch_mfma_fwd(const BandParams& p, hipStream_t st, unsigned nwg, int norm) {
   const bool bias = p.bias.p != nullptr, tau = p.tau.p != nullptr;
+  if (p.glob) {
 #ifndef TENSION_NO_GL_FWD
-  // gl_fwd keeps each lane's offset within a 64-row K / V tile in 32 bits
-  // (tile_lane); larger row strides take the band kernel's 64-bit sources
-  if (p.glob && norm == NORM_MASS_ && rows_fit_view(kTile, p.k.s1) && rows_fit_view(kTile, p.v.s1)) {
-    launch_gl_fwd(p, st);
+    // gl_fwd keeps each lane's offset within a 64-row K / V tile in 32 bits
+    // (tile_lane); larger row strides take the band kernel's 64-bit sources
+    if (rows_fit_view(kTile, p.k.s1) && rows_fit_view(kTile, p.v.s1)) {
+      launch_gl_fwd(p, st);
+      return;
+    }
+#endif
+    const BandArgs a = to_args(p);
+    if (bias) {
+      if (tau) hipLaunchKernelGGL((mfma_fwd<true, true>), dim3(nwg), dim3(kThreads), 0, st, a);
+      else hipLaunchKernelGGL((mfma_fwd<true, false>), dim3(nwg), dim3(kThreads), 0, st, a);
+    } else {
+      if (tau) hipLaunchKernelGGL((mfma_fwd<false, true>), dim3(nwg), dim3(kThreads), 0, st, a);
+      else hipLaunchKernelGGL((mfma_fwd<false, false>), dim3(nwg), dim3(kThreads), 0, st, a);
+    }
     return;
   }
-#endif
-  const bool ring = !p.glob && p.win <= kTile && p.chunk > 0;
   switch (norm) {
-    case NORM_MASS_: go_n<NORM_MASS_>(p, st, nwg, bias, tau, ring); break;
-    case NORM_COUNT_: go_n<NORM_COUNT_>(p, st, nwg, bias, tau, ring); break;
-    default: go_n<NORM_RAW>(p, st, nwg, bias, tau, ring); break;
+    case NORM_MASS_: go_n<NORM_MASS_>(p, st, bias, tau); break;
+    case NORM_COUNT_: go_n<NORM_COUNT_>(p, st, bias, tau); break;
+    default: go_n<NORM_RAW>(p, st, bias, tau); break;
   }
 }
 

@@ -53,3 +53,11 @@ def test_route_and_mixed_phases(dev, B, H, T, W, wide, norm):
     want = oracle_run({n: pick(inp[n]) for n in ("Q", "K", "V", "dO")}, W, 8.0, normalize=norm)
     for name, got, ref in zip(("out", "dQ", "dK", "dV"), (out, dq, dk, dv), (want[0], *want[2])):
         assert rel_l2(f64(pick(got)), ref) <= 4e-3, name
+
+
+def test_long_sequence(dev):
+    """All three wide kernels over 625 tiles, in segments."""
+    from bozo_amd import _lib as L
+    from tests.test_long_seq_gpu import test_window_long_sequence_segments as segments
+    segments(dev, torch.bfloat16, 40000, 1, 300, "mass")
+    assert int(L.lib().tension_last_kernel()) == L.KERNEL_MFMA
