@@ -105,15 +105,20 @@ _host = None
 
 
 def host():
-    """Load (once) and return the native call path (csrc/host.cpp)."""
+    """Load (once) and return the native call path (csrc/host.cpp).  It is
+    compiled against the installed torch, so another torch needs another build."""
     global _host
     if _host is None:
         lib()
         if not os.path.exists(HOST_PATH):
             raise TensionError(f"{HOST_PATH} is missing: build it with `python -m bozo_amd.build`")
         spec = importlib.util.spec_from_file_location("bozo_amd._host", HOST_PATH)
-        mod = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(mod)
+        try:
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+        except ImportError as e:
+            raise TensionError(f"{HOST_PATH} does not load with torch {torch.__version__} ({e}): it is bound to the torch "
+                               "it was compiled against; build it again with `python -m bozo_amd.build`") from e
         _host = mod
     return _host
 
