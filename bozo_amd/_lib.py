@@ -75,6 +75,7 @@ SIGNATURES = {
     "tension_last_error": (ctypes.c_char_p, []),
     "tension_version": (ctypes.c_char_p, []),
     "tension_last_kernel": (_i32, []),
+    "tension_last_key_groups": (_i32, []),
 }
 
 _lib = None

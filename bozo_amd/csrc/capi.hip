@@ -458,6 +458,8 @@ const char* tension_last_error(void) { return g_err.c_str(); }
 
 int tension_last_kernel(void) { return g_last_kernel; }
 
+int tension_last_key_groups(void) { return last_key_groups(); }
+
 const char* tension_version(void) { return "tension_hip 0.1 (gfx950)"; }
 
 int tension_window_fwd(const tension_buf* q, const tension_buf* k, const tension_buf* v, const tension_buf* out,

@@ -93,6 +93,8 @@ int launch_decode(int flow, int rows, bool f64, const DecodeParams& p, hipStream
 // throughout; head dim 32 or 64; phase 0 forward, 1 dQ, 2 dK / dV
 enum { SPLIT_FLOW_BF16 = 0, SPLIT_FLOW_F32 = 1, SPLIT_FLOW_F32V = 2, SPLIT_FLOW_F16 = 3 };
 int launch_split(int phase, int flow, const BandParams& p, hipStream_t st, hipError_t* err);
+// Key groups per workgroup of this thread's last split forward (0: none yet).
+int last_key_groups();
 // Compute units of the current device (queried once per device).
 int device_cus();
 int launch_rope(bool f64, const RopeParams& p, hipStream_t st, hipError_t* err);

@@ -17,6 +17,10 @@ void launch_split_fwd_f16(const BandParams& p, hipStream_t st, unsigned n);
 void launch_split_dq_f16(const BandParams& p, hipStream_t st, unsigned n);
 void launch_split_dkv_f16(const BandParams& p, hipStream_t st, unsigned n);
 
+static thread_local int g_key_groups = 0;
+
+int last_key_groups() { return g_key_groups; }
+
 int launch_split(int phase, int flow, const BandParams& p_in, hipStream_t st, hipError_t* err) {
   if (flow < SPLIT_FLOW_BF16 || flow > SPLIT_FLOW_F16) return -1;
   if (phase < 0 || phase > 2) return -1;
@@ -60,13 +64,14 @@ int launch_split(int phase, int flow, const BandParams& p_in, hipStream_t st, hi
       nwg = bh * runs;
     }
   }
-  // a forward whose bands span more than two key blocks, on a grid of at most one
+  // a forward whose windows are wider than a key block, on a grid of at most one
   // workgroup per CU: two key groups per workgroup (p.chunk < 0, xb_fwd).  B1
   // H16 T1024, autocast / float32: W256 14.5 -> 12.6 / 18.0 -> 15.9 us, with tau
   // 20.2 -> 17.7 / 23.7 -> 20.1, global 36.6 -> 27.6 / 47.9 -> 36.8; past one per
   // CU the larger workgroups no longer all fit at once (B2 H12 T1024 with tau
   // 25.8 -> 31.8 / 30.4 -> 35.8)
   if (phase == 0 && (p.glob || p.win > 64) && nwg <= device_cus()) p.chunk = -1;
+  if (phase == 0) g_key_groups = p.chunk < 0 ? 2 : 1;
   const unsigned n = (unsigned)nwg;
   typedef void (*Launch)(const BandParams&, hipStream_t, unsigned);
   static const Launch table[4][3] = {

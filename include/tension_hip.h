@@ -365,6 +365,10 @@ enum {
 };
 int tension_last_kernel(void);
 
+/* Key groups per workgroup of the last split-kernel forward launched on the
+ * calling thread: 1, or 2 where a small grid takes two (0 before the first). */
+int tension_last_key_groups(void);
+
 #ifdef __cplusplus
 }
 #endif
