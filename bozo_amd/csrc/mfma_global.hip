@@ -105,8 +105,9 @@ __device__ __forceinline__ int gl_opaque(int lane) {
 // switch for all N, and branch-free loads (a pair without a slot reads column 0 and
 // is masked), so they are in flight together: with a switch and a wait for each
 // pair a block with columns was a chain of sixteen loads.  With these, gl_opaque
-// and the blocks with columns in loops of their own, gl_fwd and gl_dq with tau_local
-// run at three waves per SIMD like those without it: B8 H12 T1024, Wl 64: gl_fwd
+// and, in gl_dq and gl_dkv, the blocks with columns in loops of their own, gl_fwd
+// and gl_dq with tau_local run at three waves per SIMD like those without it (2 and
+// 4 registers spilled; gl_dkv with a bias and dtau_local, at two waves, 8): B8 H12 T1024, Wl 64: gl_fwd
 // 32.5 -> 29.1 us, gl_dq 47.9 -> 43.4, gl_dkv 58.1 -> 52.1; forward + backward
 // B4 H12 T2048: Wl 64 198 -> 177 us, Wl 512 256 -> 206 us.
 template <int N, typename E, typename Row, typename Col>
@@ -150,7 +151,6 @@ __device__ __forceinline__ void gl_tau_put8(const Buf& b, int64_t off, int col0,
 #define TENSION_GL_FWD_WPE 3
 #endif
 // with a bias the per-pair operands need more registers: two waves per SIMD
-// instead of spilling
 #ifndef TENSION_GL_FWD_WPE_OPT
 #define TENSION_GL_FWD_WPE_OPT 2
 #endif

@@ -1479,7 +1479,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NT == 
 // starts), and the second read is an L2 hit.
 // With a float32 V the register budget is stated: left to the compiler the kernel
 // took 272 registers, one wave per SIMD, and one tile per workgroup was faster
-// (B8 H12 T1000 d64 W64: 54 us; the runs at two waves 45 us).  So is that of the
+// (B8 H12 T1000 d64 W64: 54 us; the runs at two waves, with 4 to 6 registers
+// spilled, 45 us).  So is that of the
 // float16 kernels at head dim 32 with a dTau or a bias, which the compiler left
 // 2 to 4 registers above three waves: one run per (b, h) from 513 (b, h) on, more
 // than two workgroups per CU (B40 H16 T256 W33, valid count, dTau 41.5 -> 32.9 us;

@@ -408,8 +408,9 @@ def rope(x: Tensor, cos: Tensor, sin: Tensor, pos_offset: int = 0,
 # global_fwd / global_bwd, rope) with fake-tensor shape functions and
 # autograd formulas, so torch.compile traces a model through them without a
 # graph break (the reference compiles its model, train.py:776-780).  The
-# public functions call them while torch.compile traces and the autograd
-# Functions above in eager mode.
+# public functions call them while torch.compile traces; eager calls take the
+# native autograd nodes (csrc/host.cpp), tracing and functorch transforms the
+# autograd Functions above.
 
 @torch.library.custom_op("bozo::window_fwd", mutates_args=(), device_types="cuda")
 def _op_window_fwd(Q: Tensor, K: Tensor, V: Tensor, window: int, scale: float, return_tau: bool,
