@@ -49,14 +49,17 @@ int launch_split(int phase, int flow, const BandParams& p_in, hipStream_t st, hi
     if (phase == 2 && flow == SPLIT_FLOW_F32V && p.D == 64) {
       // the float32 kernel holds exactly two workgroups per CU, so a few runs over
       // would be a round of their own, and the runs are worth it only where they
-      // fill their rounds: to 65%, with a bias or a dTau (where they gain less over
-      // one tile per workgroup) to 90%.  One tile -> runs, valid count, W 64, us:
+      // fill their rounds: to 60%, with a bias or a dTau (where they gain less over
+      // one tile per workgroup) to 90%, to 75% when a run has four tiles at most (an
+      // empty place costs little).  One tile -> runs, valid count, W 64, us:
       // 96 (b, h) of T1000 51 -> 45, with dTau 59 -> 58; 128 64 -> 54, 75 -> 69; 192
       // (three runs each, 2.25 per CU) 88 -> 99, 104 -> 135; 514 220 -> 269, 251 ->
-      // 374; 704 of T256 83 -> 77, 99 -> 102; 1024 117 -> 100, 140 -> 124.
+      // 374; of T256, 704 83 -> 77, 99 -> 102; 448 59 -> 49, 70 -> 63; 1024 117 -> 100,
+      // 140 -> 124.
       runs = slots / bh;
       const int64_t wg = bh * (runs < 1 ? 1 : runs), rounds = (wg + slots - 1) / slots;
-      take = 20 * wg >= (p.dtau.p || p.bias.p ? 18 : 13) * rounds * slots;
+      const bool side = p.dtau.p || p.bias.p;
+      take = 20 * wg >= (!side ? 12 : p.ntiles <= 4 ? 15 : 18) * rounds * slots;
     }
     if (runs < 1) runs = 1;
     if (take && runs < p.ntiles) {
