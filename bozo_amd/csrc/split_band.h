@@ -41,6 +41,7 @@
 
 #include <type_traits>
 
+#include "kernels.h"
 #include "mfma_common.h"
 
 namespace tension {
@@ -617,6 +618,11 @@ struct FwdTile {
 // waves per SIMD, what its LDS admits), where the compiler left them at three:
 // float16 B8 H12 T1024 global with tau_local 98 -> 91 us, B4 H16 T1024 W256 with
 // tau 44 -> 37, with a bias 61 -> 46; bf16 with a bias 52 -> 40.
+// Where the fourth workgroup on a CU would not save a round of them, a local
+// window's are held at three by LDS they do not use (float16 B8 H12 T1024 W400,
+// two rounds of 1536 workgroups either way: 91.5 -> 88.0 us; the global block,
+// whose tiles differ in length, gains from the fourth as often as it loses).
+constexpr unsigned kFwdThreePerCu = 12 * 1024;  // + 40 KB: three to a CU's 160 KB
 constexpr int fwd_waves(int NT, int D, bool bias, bool tau, int ks) {
   return ks == 1 && D == 64 && tau && (NT == 2 || (NT == 1 && bias)) ? 4 : 1;
 }
@@ -1569,14 +1575,15 @@ void launch_norm(const BandParams& p, hipStream_t st, unsigned n) {
   const bool bias = p.bias.p != nullptr;
   const dim3 grid(n), block(kThreads);
   const BandArgs a = to_args(p);
+  unsigned dyn = 0;  // dynamic LDS
 #define XB_BT(K, ...)                                                                           \
   do {                                                                                          \
     if (bias) {                                                                                 \
-      if (opt) hipLaunchKernelGGL((K<NT, NV, D, NORM, true, true __VA_ARGS__>), grid, block, 0, st, a);  \
-      else hipLaunchKernelGGL((K<NT, NV, D, NORM, true, false __VA_ARGS__>), grid, block, 0, st, a);     \
+      if (opt) hipLaunchKernelGGL((K<NT, NV, D, NORM, true, true __VA_ARGS__>), grid, block, dyn, st, a);  \
+      else hipLaunchKernelGGL((K<NT, NV, D, NORM, true, false __VA_ARGS__>), grid, block, dyn, st, a);     \
     } else {                                                                                    \
-      if (opt) hipLaunchKernelGGL((K<NT, NV, D, NORM, false, true __VA_ARGS__>), grid, block, 0, st, a); \
-      else hipLaunchKernelGGL((K<NT, NV, D, NORM, false, false __VA_ARGS__>), grid, block, 0, st, a);    \
+      if (opt) hipLaunchKernelGGL((K<NT, NV, D, NORM, false, true __VA_ARGS__>), grid, block, dyn, st, a); \
+      else hipLaunchKernelGGL((K<NT, NV, D, NORM, false, false __VA_ARGS__>), grid, block, dyn, st, a);    \
     }                                                                                           \
   } while (0)
   if constexpr (PHASE == 0) {
@@ -1587,6 +1594,11 @@ void launch_norm(const BandParams& p, hipStream_t st, unsigned n) {
       const dim3 block(2 * kThreads);
       XB_BT(xb_fwd, , 2);
     } else {
+      if (!p.glob && fwd_waves(NT, D, bias, opt, 1) == 4) {
+        // four workgroups on a CU only where they save a round over three
+        const int64_t cus = device_cus();
+        if ((n + 4 * cus - 1) / (4 * cus) == (n + 3 * cus - 1) / (3 * cus)) dyn = kFwdThreePerCu;
+      }
       XB_BT(xb_fwd, , 1);
     }
   } else if constexpr (PHASE == 1) {
