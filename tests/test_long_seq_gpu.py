@@ -10,7 +10,7 @@ full-length HIP run.  Segments sit at the start, in the middle (not aligned
 to the 64-row tiles, crossing the fused backward's run boundaries) and at
 the end of the sequence.  The paths: the fused backward's fast path (W = 64,
 T a multiple of 64), its general path (ragged T), the split backward
-(W > 64) and the float32 exact kernels.  The global block has no such
+(W > 64) and the float32 split kernels.  The global block has no such
 locality; it is checked whole at T = 3000 (ragged, 47 tiles).
 
 Tolerances as elsewhere: bf16 relative L2 2e-2 over the checked rows,
@@ -37,7 +37,7 @@ def _segments(T, W):
     (torch.bfloat16, 65536, 3, 64, "mass"),      # fused backward, fast path
     (torch.bfloat16, 65573, 2, 64, "count"),     # fused backward, ragged T
     (torch.bfloat16, 40000, 2, 100, "mass"),     # split backward (W > 64)
-    (torch.float32, 20000, 2, 64, "mass"),       # exact kernels
+    (torch.float32, 20000, 2, 64, "mass"),       # split kernels, three terms
 ])
 def test_window_long_sequence_segments(dev, dtype, T, H, W, norm):
     D = 64
