@@ -25,8 +25,7 @@ __global__ __launch_bounds__(kThreads) void mfma_bwd_dkv(BandArgs args) {
   __shared__ float sa[kTile], sc[kTile];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 4, c = lane & 15;
-  // key tile 0 sees the most queries in the global band: natural order is
-  // already heaviest first
+  // local windows: every full tile sees as many queries, natural order
   const TileId id = tile_id(p, false);
   const int b = id.b, h = id.h, T = p.T;
   const int k0 = id.tile * kTile;
